@@ -10,8 +10,8 @@
 // vertex unknowns -1).  The factorisation is right-looking and blocked by
 // NB = 256:
 //   1. k_diag_factor: one workgroup factors the NB x NB diagonal block
-//      (inner blocks of 32 in LDS), writes the signs and the explicit
-//      inverse of the diagonal L block;
+//      (16 x 16 tiles in MFMA accumulators) and writes the signs;
+//      k_diag_inverse forms the explicit inverse of the diagonal L block;
 //   2. panel X = A21 * Linv^T (MFMA GEMM), L21 = X * S1;
 //   3. trailing update A22 -= X * L21^T on the lower triangle (MFMA GEMM).
 // Triangular solves with many right-hand sides use the stored diagonal
@@ -560,374 +560,436 @@ __global__ void __launch_bounds__(256) k_gemm_grouped(const GemmDesc* __restrict
 
 // ---------------------------------------------------------------------------
 // diagonal block: signed Cholesky A11 = L11 S1 L11^T and Linv = L11^-1.
-// Both kernels are latency bound (one NB x NB block, about 11 MFLOP), so
-// they are built to keep the serial chain short.
-// k_diag_factor: one workgroup; inner panels of IB = 32 columns:
-//   1. the panel (rows c0.., IB columns) is read into LDS, transposed;
-//   2. one wave factors the IB x IB pivot block in registers (lane i holds
-//      the symmetric row i, row j is broadcast with readlane, so the 32
-//      pivot steps need no workgroup barrier) and inverts it by forward
-//      substitution (lane j holds column j of the inverse Mi);
-//   3. the rows below: L_r = A_r Mi^T S1 (one thread per row);
-//   4. the rest of the block -= L S L^T (4 x 4 register tiles over the lower
-//      triangle; A is read and written in global memory, L2 resident).
-// The IB x IB inverses are stored as the diagonal IB-blocks of Linv.
-// k_diag_inverse: one workgroup per IB-column block c of Linv; the column
-// block is built in LDS by block forward substitution from those inverses:
-// X_rc = -Mi_r sum_{c <= q < r} L_rq X_qc.
+// Both kernels are latency bound (one NB x NB block, about 11 MFLOP on one
+// CU, on the critical path of every factorisation), so they keep the block in
+// MFMA accumulators and the serial chain short.  Unit: 16 x 16 tiles.
+// k_diag_factor: one workgroup of 8 waves.  Wave 0 owns the diagonal tiles,
+// the others the tiles below the diagonal (column-major order, dealt in
+// turn, so every tile column is spread over all of them).  A tile (i, j) is
+// held transposed, T = A_ij^T: an accumulator of T is then the B operand of
+// the next product as it stands (the k order inside a product is the
+// accumulator's row order, for both operands), and X_ij^T is the A operand
+// of another tile.  Step p:
+//   1. wave 0 has factored the pivot tile in registers (pivot_tile: row j is
+//      broadcast inside 16-lane groups, no LDS and no barrier on the pivot
+//      chain) and stored Mi = L_pp^-1 as an A operand;
+//   2. the tiles below it: X^T = Mi T (four MFMAs), to LDS and L = X S to A;
+//   3. T_ij -= X_j S X_i^T for the tiles right of column p; wave 0 updates
+//      the next pivot tile first and factors it while the others update.
+// The 16 x 16 inverses are stored as the diagonal tiles of Linv.
+// k_diag_inverse: one workgroup of 4 waves per 16-column block c of Linv;
+// right-looking block forward substitution X_q = -Mi_q acc_q,
+// acc_r += L_rq X_q, the accumulators in registers again.
+// Measured on a 256-block: factor 49 us FP32 and 58 us FP64 (inner panels of
+// 32 columns with LDS products and the trailing part in global memory: 250
+// and 341 us), about 2900 / 3500 cycles a pivot tile and 1000-1500 cycles of
+// barriers and X^T a step; inverse 18 us (45 us FP32, 51 us FP64).  Beside an
+// FP64 update, whose two workgroups a CU leave no room for its registers,
+// the FP64 factor takes 400 us (666 us).
 // ---------------------------------------------------------------------------
-constexpr int IB = 32;
-constexpr int DF_THREADS = 256;     // factor: one wave per SIMD, so that the
-                                    // workgroup fits beside a running GEMM
-                                    // workgroup on one CU
-constexpr int DIAG_THREADS = 512;   // inverse
-constexpr int PT_LD = FACT_NB + 4;   // row stride of the transposed panel (16-byte rows)
-constexpr int DT_TILES = 4;          // trailing 4 x 4 tiles per thread and pass
+constexpr int BT = 16;                       // tile of the diagonal block
+constexpr int DF_THREADS = 512;              // factor
+constexpr int DF_WAVES = DF_THREADS / 64;
+constexpr int DF_TILES = FACT_NB / BT;       // tiles along the block
+constexpr int DF_SLOTS = (DF_TILES * (DF_TILES - 1) / 2 + DF_WAVES - 2) / (DF_WAVES - 1);   // tiles of a wave
+constexpr int DIAG_THREADS = 256;            // inverse
+constexpr int INV_SLOTS = DF_TILES / (DIAG_THREADS / 64);
 
-__device__ __forceinline__ float lane_read(float v, int src) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src));
-}
-__device__ __forceinline__ double lane_read(double v, int src) {
-    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, src);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), src);
-    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+// value of lane j of the caller's 16-lane group, in every lane of the group
+template <int J, typename T>
+__device__ __forceinline__ T group_bcast(T v) {
+    return __builtin_amdgcn_update_dpp(v, v, 0x150 + J, 0xf, 0xf, true);
 }
 
-// four consecutive LDS values (16-byte aligned for float, 32 for double)
-__device__ __forceinline__ void lds4(const float* p, float (&v)[4]) {
-    const float4 q = *(const float4*)p;
-    v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+// a += n * (a of lane j of the 16-lane group), one instruction.  The DPP read
+// of a needs two wait states after the write of a: callers keep at least two
+// instructions between them.
+template <int J>
+__device__ __forceinline__ void fmac_bcast(float& a, float n) {
+    asm volatile("v_fmac_f32_dpp %0, %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf" : "+v"(a) : "v"(n), "n"(J));
 }
-__device__ __forceinline__ void lds4(const double* p, double (&v)[4]) {
-    const double2 q0 = *(const double2*)p, q1 = *(const double2*)(p + 2);
-    v[0] = q0.x; v[1] = q0.y; v[2] = q1.x; v[3] = q1.y;
+template <int J>
+__device__ __forceinline__ void fmac_bcast(double& a, double n) {
+    asm volatile("v_fmac_f64_dpp %0, %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf" : "+v"(a) : "v"(n), "n"(J));
 }
 
-// Step 2 (wave 0).  Pt[l][i] (l, i < IB) holds the symmetric pivot block,
-// padded with the identity beyond w.  Lanes 0..31 hold rows; lanes 32..63
-// repeat them and store nothing.  L replaces the pivot block in Pt (row i
-// in Pt[.][i]; entries above the diagonal are not meaningful) and is also
-// kept row-major in Ls; Mi = L^-1 is stored row-major.
-template <typename T>
-__device__ __forceinline__ void pivot_block(T (*Pt)[PT_LD], int w, T (*Mi)[IB], T (*Ls)[IB + 4], T* __restrict__ sg,
-                                            T* __restrict__ ig, int* __restrict__ info, int64_t kglob, T tiny) {
-    const int lane = threadIdx.x & 63;
-    int i = lane & (IB - 1);
-    asm volatile("" : "+v"(i));   // keeps per-lane selects inside the panel loop
-    T a[IB];
+// 1/d within about an ulp (the hardware estimate and a Newton step, cubic for
+// FP64): the IEEE division's scaling steps would double the pivot chain
+__device__ __forceinline__ float pivot_rcp(float d) {
+    const float y = __builtin_amdgcn_rcpf(d);
+    return fmaf(y, fmaf(-d, y, 1.f), y);
+}
+__device__ __forceinline__ double pivot_rcp(double d) {
+    const double y = __builtin_amdgcn_rcp(d);
+    const double e = fma(-d, y, 1.0);
+    return fma(y, fma(e, e, e), y);
+}
+
+// sqrt(x) and 1/sqrt(x), x > 0: the hardware estimate, a Newton step (cubic
+// for FP64), and the root's residual once more
+__device__ __forceinline__ void pivot_root(float x, float& r, float& g) {
+    const float y = __builtin_amdgcn_rsqf(x);
+    g = fmaf(0.5f * y, fmaf(-x * y, y, 1.f), y);
+    const float q = x * g;
+    r = fmaf(fmaf(-q, q, x), 0.5f * g, q);
+}
+__device__ __forceinline__ void pivot_root(double x, double& r, double& g) {
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-x * y, y, 1.0);
+    g = fma(y * e, fma(e, 0.375, 0.5), y);
+    const double q = x * g;
+    r = fma(fma(-q, q, x), 0.5 * g, q);
+}
+
+// Pivots J, J + 1, .. of a tile: lane = row i (of 16) in each of four groups;
+// every group holds the whole row a, group q the four columns
+// Acc::row(lane, .) of the unit inverse b.  Rows below J lose f times row J;
+// a[J] keeps f = Lu(i, J).  iw = min(i, w): pivots from w on change nothing.
+// The chain bcast, reciprocal, f, a[J + 1] is the latency; the rest of the
+// row fills it.
+template <typename T, int J>
+struct PivotStep {
+    static __device__ __forceinline__ void run(T (&a)[BT], T (&b)[4], int iw, T& dsave) {
+        const T d = group_bcast<J>(a[J]);
+        if (iw >= J) dsave = d;          // the last one written is the row's own
+        const T q = a[J] * pivot_rcp(d);
+        const T nf = iw > J ? -q : T(0);
+        // nf's chain is more than two instructions behind the last fmac
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int l = 0; l < IB; ++l) a[l] = Pt[l][i];
-    // right-looking, one pivot per step: with a = column j after the
-    // previous steps and d = a_j, A(i,l) -= a_i a_l / d and
-    // L(i,j) = a_i / (sqrt|d| s_j), s_j = sign(d)
-    // (one reciprocal and one square root per step: 1/(sqrt|d| s) = sqrt|d| / d)
-    int bad = -1;
+        for (int l = J + 1; l < BT; ++l) fmac_bcast<J>(a[l], nf);
 #pragma unroll
-    for (int j = 0; j < IB; ++j) {
-        const T d = lane_read(a[j], j);
-        const T s = d >= T(0) ? T(1) : T(-1);
-        const T id = T(1) / d;
-        const T r = sqrt(fabs(d));
-        const T g = r * id;
-        const T f = a[j] * id;
-#pragma unroll
-        for (int l = j + 1; l < IB; ++l) a[l] -= f * lane_read(a[l], j);
-        a[j] = (i == j) ? r : a[j] * g;
-        if (lane == 0) ig[j] = s * g;   // 1 / L(j, j)
-        if (j < w) {
-            if (lane == 0) sg[j] = s;
-            if (bad < 0 && !(fabs(d) > tiny)) bad = j;
-        }
+        for (int c = 0; c < 4; ++c) fmac_bcast<J>(b[c], nf);
+        a[J] = q;                        // rows up to J: not read again
+        __builtin_amdgcn_sched_barrier(0);
+        PivotStep<T, J + 1>::run(a, b, iw, dsave);
     }
-    // L to LDS (row i of L in Ls[i][.] for the substitution, in Pt[.][i]
-    // for the stores)
-    if (lane < IB) {
+};
+template <typename T>
+struct PivotStep<T, BT> {
+    static __device__ __forceinline__ void run(T (&)[BT], T (&)[4], int, T&) {}
+};
+
+// Signed Cholesky of the pivot tile P (both halves valid; rows and columns
+// from w on arbitrary), by one wave: Lu D Lu^T without square roots, then
+// L = Lu sqrt|D|, S = sign D, Mi = |D|^-1/2 Lu^-1.  Mi goes to mi in the A
+// operand layout and to Linv, the lower half of L to A, the signs to sg and
+// sgn; rt is scratch.
+template <typename T>
+__device__ __forceinline__ void pivot_tile(const T (*P)[BT + 1], int w, T (*mi)[64], T* __restrict__ sg,
+                                           T* __restrict__ rt, T* __restrict__ sgn, T* __restrict__ A, int64_t lda,
+                                           T* __restrict__ Linv, int64_t ldl, int* __restrict__ info, int64_t kglob,
+                                           T tiny) {
+    const int lane = threadIdx.x & 63;
+    int i = lane & 15;
+    asm volatile("" : "+v"(i));   // the lane masks are formed here, not kept over the panel loop
+    T a[BT], b[4], d = T(1);
 #pragma unroll
-        for (int l = 0; l < IB; ++l) {
-            Ls[i][l] = a[l];
-            Pt[l][i] = a[l];
-        }
+    for (int l = 0; l < BT; ++l) a[l] = P[i][l];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) b[c] = Acc<T>::row(lane, c) == i ? T(1) : T(0);
+    PivotStep<T, 0>::run(a, b, min(i, w), d);
+    T r, g;
+    pivot_root(fabs(d), r, g);
+    if (lane < BT) {
+        const T s = d >= T(0) ? T(1) : T(-1);
+        sg[lane] = s;
+        rt[lane] = r;
+        if (lane < w) sgn[lane] = s;
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // Mi = L^-1 by forward substitution, lane i holds column i
-    T x[IB];
 #pragma unroll
-    for (int r = 0; r < IB; ++r) {
-        T acc0 = (r == i) ? T(1) : T(0), acc1 = T(0);
-#pragma unroll
-        for (int l = 0; l < r; ++l) {
-            if (l & 1) acc1 -= Ls[r][l] * x[l];
-            else acc0 -= Ls[r][l] * x[l];
-        }
-        x[r] = (acc0 + acc1) * ig[r];
+    for (int c = 0; c < 4; ++c) {
+        const T v = b[c] * g;
+        mi[c][lane] = v;
+        const int col = Acc<T>::row(lane, c);
+        if (i < w && col < w) Linv[i + (int64_t)col * ldl] = v;
     }
-    if (lane < IB) {
+    // column 4 c + group of L: f sqrt|d| of the column
+    const int q = lane >> 4;
 #pragma unroll
-        for (int r = 0; r < IB; ++r) Mi[r][i] = x[r];
+    for (int c = 0; c < 4; ++c) {
+        const int l = 4 * c + q;
+        const T rl = rt[l];
+        const T f0 = a[4 * c], f1 = a[4 * c + 1], f2 = a[4 * c + 2], f3 = a[4 * c + 3];
+        const T lo = q & 1 ? f1 : f0, hi = q & 1 ? f3 : f2;
+        const T f = q & 2 ? hi : lo;
+        if (l <= i && i < w) A[i + (int64_t)l * lda] = l == i ? rl : f * rl;
     }
-    if (lane == 0 && bad >= 0 && info[0] == 0) info[0] = (int)(kglob + bad + 1);
+    const unsigned long long bad = __ballot(lane < w && !(fabs(d) > tiny));
+    if (bad && lane == 0 && info[0] == 0) info[0] = (int)(kglob + __ffsll(bad));
 }
 
 template <typename T>
 __device__ __forceinline__ void diag_body(T* __restrict__ A11, int64_t lda, int nb, T* __restrict__ sgn,
                                           int* __restrict__ info, int64_t k0, T tiny, T* __restrict__ Linv,
                                           int64_t ldl) {
-    __shared__ __align__(16) T Pt[IB][PT_LD];
-    __shared__ T Mi[IB][IB];
-    __shared__ __align__(16) T Ls[IB][IB + 4];
-    __shared__ T sg[IB];
-    __shared__ T ig[IB];
-    const int tid = threadIdx.x;
-    for (int c0 = 0; c0 < nb; c0 += IB) {
-        const int w = min(IB, nb - c0);
-        const int m = nb - c0;
-        // 1. panel into LDS; the pivot block is mirrored (its part above the
-        // diagonal in A is stale) and padded with the identity
-        for (int e = tid; e < m * w; e += DF_THREADS) {
-            const int r = e % m, l = e / m;
-            if (r < l) continue;
-            const T v = A11[(c0 + r) + (int64_t)(c0 + l) * lda];
-            Pt[l][r] = v;
-            if (r < w) Pt[r][l] = v;
+    typedef typename Acc<T>::type acc_t;
+    __shared__ T panel[DF_TILES][4][64];   // X of the tile column, operand layout
+    __shared__ T diag[DF_TILES][4][64];    // the diagonal tiles, accumulator layout
+    __shared__ T mi[4][64];
+    __shared__ T piv[BT][BT + 1];
+    __shared__ T sg[BT], rt[BT];
+    __builtin_amdgcn_s_setprio(2);         // the critical path, beside a trailing update
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int np = (nb + BT - 1) / BT;
+    const int li = lane & 15;
+    // element r of the caller's lane of tile (i, j), the stored half of a
+    // diagonal tile mirrored.  Indices beyond nb are clamped and the value is
+    // not masked (the compiler would branch around each load and wait for
+    // it): what they bring reaches only rows and pivots beyond nb, which
+    // nothing stores and no stored row depends on.
+    auto load = [&](int i, int j, int r) -> T {
+        const int row = min(BT * i + li, nb - 1), col = min(BT * j + Acc<T>::row(lane, r), nb - 1);
+        return A11[max(row, col) + (int64_t)min(row, col) * lda];
+    };
+    T ns[4];   // minus the signs of step p, by the lane's rows of an accumulator
+    auto read_signs = [&] {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) ns[r] = -sg[Acc<T>::row(lane, r)];
+    };
+    // diagonal tile i of the step's update (the next pivot tile is wave 0's,
+    // the later ones are dealt over all waves)
+    auto update_diag = [&](int i) {
+        acc_t t;
+        T x[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            t[r] = diag[i][r][lane];
+            x[r] = panel[i][r][lane];
         }
-        if (w < IB) {
-            for (int e = tid; e < IB * IB; e += DF_THREADS) {
-                const int r = e % IB, l = e / IB;
-                if (r >= w || l >= w) Pt[l][r] = (r == l) ? T(1) : T(0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) t = Acc<T>::mfma(x[r] * ns[r], x[r], t);
+        return t;
+    };
+    auto update_diags = [&](int p) {
+        for (int i = (p + 2) / DF_WAVES * DF_WAVES + wave; i < np; i += DF_WAVES) {
+            if (i < p + 2) continue;
+            const acc_t u = update_diag(i);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) diag[i][r][lane] = u[r];
+        }
+    };
+    static_assert(DF_TILES == 2 * DF_WAVES, "two diagonal tiles a wave");
+    {
+        T d0[4], d1[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            d0[r] = load(wave, wave, r);
+            d1[r] = load(wave + DF_WAVES, wave + DF_WAVES, r);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            diag[wave][r][lane] = d0[r];
+            diag[wave + DF_WAVES][r][lane] = d1[r];
+        }
+    }
+    if (wave == 0) {
+        __builtin_amdgcn_s_setprio(3);     // the pivots, beside this block's updates
+        acc_t t;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) t[r] = diag[0][r][lane];
+        for (int p = 0;; ++p) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) piv[Acc<T>::row(lane, r)][li] = t[r];
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            const int c = BT * p;
+            pivot_tile<T>(piv, min(BT, nb - c), mi, sg, rt, sgn + k0 + c, A11 + c + (int64_t)c * lda, lda,
+                          Linv + c + (int64_t)c * ldl, ldl, info, k0 + c, tiny);
+            if (p > 0) update_diags(p - 1);
+            __syncthreads();   // Mi and the signs of step p, the panel buffer free
+            if (p + 1 == np) return;
+            read_signs();
+            __syncthreads();   // the panel is complete, Mi and the signs are read
+            t = update_diag(p + 1);
+        }
+    }
+    // the wave's tiles and their columns; empty slots come last, count as
+    // active at every step and update what nothing reads
+    acc_t acc[DF_SLOTS];
+    int ti[DF_SLOTS], tj[DF_SLOTS];
+    {
+        int i = wave, j = 0;
+#pragma unroll
+        for (int s = 0; s < DF_SLOTS; ++s) {
+            if (s > 0) i += DF_WAVES - 1;
+            while (j < np && i >= np) {      // past the column's end: to the next column
+                i += j + 2 - np;
+                ++j;
             }
+            const bool in = j < np;
+            ti[s] = in ? i : 0;
+            tj[s] = in ? j : DF_TILES;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[s][r] = load(ti[s], tj[s], r);
+            __builtin_amdgcn_sched_barrier(0);   // one tile's addresses at a time
+        }
+    }
+    // a tile index the compiler forms no address from ahead of its use (the
+    // addresses of every slot, kept over the loop, would spill the tiles)
+    auto fresh = [](int v) {
+        asm volatile("" : "+s"(v));
+        return v;
+    };
+    for (int p = 0;; ++p) {
+        __syncthreads();
+        if (p + 1 == np) return;
+        T m[4];
+        read_signs();
+#pragma unroll
+        for (int r = 0; r < 4; ++r) m[r] = mi[r][lane];
+#pragma unroll
+        for (int s = 0; s < DF_SLOTS; ++s) {
+            if (tj[s] != p) continue;
+            const int t = fresh(ti[s]);
+            acc_t x = {0, 0, 0, 0};
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x = Acc<T>::mfma(m[r], acc[s][r], x);
+            acc[s] = x;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) panel[t][r][lane] = x[r];
         }
         __syncthreads();
-        // 2. pivot block
-        if (tid < 64) pivot_block<T>(Pt, w, Mi, Ls, sg, ig, info, k0 + c0, tiny);
-        __syncthreads();
-        for (int e = tid; e < IB * IB; e += DF_THREADS) {
-            const int r = e % IB, j = e / IB;
-            if (r < w && j < w) {
-                Linv[(c0 + r) + (int64_t)(c0 + j) * ldl] = Mi[r][j];
-                if (r >= j) A11[(c0 + r) + (int64_t)(c0 + j) * lda] = Pt[j][r];
+        // two tiles at a time, so that one's products fill the other's
+        // latency; activity grows with the slot
+        static_assert(DF_SLOTS % 2 == 0, "slots go in pairs");
+        auto operands = [&](int s, T (&x)[4], T (&y)[4]) {
+            const int i = fresh(ti[s]), j = fresh(tj[s]) & (DF_TILES - 1);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                x[r] = panel[j][r][lane] * ns[r];
+                y[r] = panel[i][r][lane];
             }
-        }
-        if (tid < w) sgn[k0 + c0 + tid] = sg[tid];
-        if (m <= w) break;   // last inner panel (w == IB otherwise)
-        // 3. rows below, one thread per row: L(r, j) = s_j sum_{l <= j}
-        // A(r, l) Mi(j, l).  Pt keeps L s.
-        const int mt = m - IB;
-        for (int rl = tid; rl < mt; rl += DF_THREADS) {
-            T row[IB];
+        };
 #pragma unroll
-            for (int l = 0; l < IB; ++l) row[l] = Pt[l][IB + rl];
-#pragma unroll 2
-            for (int j = 0; j < IB; ++j) {
-                T acc0 = 0, acc1 = 0;   // Mi(j, l) = 0 for l > j
+        for (int s = 0; s < DF_SLOTS; s += 2) {
+            if (tj[s + 1] <= p) continue;
+            T x0[4], y0[4], x1[4], y1[4];
+            operands(s + 1, x1, y1);
+            if (tj[s] > p) {
+                operands(s, x0, y0);
 #pragma unroll
-                for (int l = 0; l < IB; l += 2) {
-                    acc0 += row[l] * Mi[j][l];
-                    acc1 += row[l + 1] * Mi[j][l + 1];
+                for (int r = 0; r < 4; ++r) {
+                    acc[s] = Acc<T>::mfma(x0[r], y0[r], acc[s]);
+                    acc[s + 1] = Acc<T>::mfma(x1[r], y1[r], acc[s + 1]);
                 }
-                const T acc = acc0 + acc1;
-                A11[(c0 + IB + rl) + (int64_t)(c0 + j) * lda] = acc * sg[j];
-                Pt[j][IB + rl] = acc;
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[s + 1] = Acc<T>::mfma(x1[r], y1[r], acc[s + 1]);
             }
         }
-        __syncthreads();
-        // 4. trailing lower triangle, rows and columns IB.. of the panel
-        const int nt = (mt + 3) >> 2;
-        const int ntri = nt * (nt + 1) / 2;
-        for (int t0 = 0; t0 < ntri; t0 += DF_THREADS * DT_TILES) {
-            T acc[DT_TILES][4][4];
-            int R[DT_TILES], C[DT_TILES];
+        update_diags(p);
+        // L of the panel, off the way to the update
 #pragma unroll
-            for (int u = 0; u < DT_TILES; ++u) {
-                const int t = t0 + u * DF_THREADS + tid;
-                int rr = -1, cc = 0;
-                if (t < ntri) {
-                    // t = q (q + 1) / 2 + p, p <= q: tile (nt-1-p, nt-1-q), so
-                    // that consecutive lanes take consecutive row tiles
-                    int q = (int)((sqrtf(8.f * (float)t + 1.f) - 1.f) * 0.5f);
-                    while (q * (q + 1) / 2 > t) --q;
-                    while ((q + 1) * (q + 2) / 2 <= t) ++q;
-                    rr = nt - 1 - (t - q * (q + 1) / 2);
-                    cc = nt - 1 - q;
-                }
-                R[u] = rr;
-                C[u] = cc;
+        for (int s = 0; s < DF_SLOTS; ++s) {
+            if (tj[s] != p) continue;
+            const int row = BT * fresh(ti[s]) + li;
+            if (row < nb) {
 #pragma unroll
-                for (int a = 0; a < 4; ++a)
-#pragma unroll
-                    for (int b = 0; b < 4; ++b) {
-                        const int r = 4 * rr + a, c = 4 * cc + b;
-                        acc[u][a][b] = (rr >= 0 && r < mt && r >= c)
-                                           ? A11[(c0 + IB + r) + (int64_t)(c0 + IB + c) * lda]
-                                           : T(0);
-                    }
-            }
-#pragma unroll
-            for (int u = 0; u < DT_TILES; ++u) {
-                if (R[u] < 0) continue;
-#pragma unroll 8
-                for (int j = 0; j < IB; ++j) {
-                    T x[4], y[4];
-                    lds4(&Pt[j][IB + 4 * R[u]], x);
-                    lds4(&Pt[j][IB + 4 * C[u]], y);
-                    const T s = sg[j];
-#pragma unroll
-                    for (int b = 0; b < 4; ++b) y[b] *= s;
-#pragma unroll
-                    for (int a = 0; a < 4; ++a)
-#pragma unroll
-                        for (int b = 0; b < 4; ++b) acc[u][a][b] -= x[a] * y[b];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < DT_TILES; ++u) {
-                const int rr = R[u], cc = C[u];
-#pragma unroll
-                for (int a = 0; a < 4; ++a)
-#pragma unroll
-                    for (int b = 0; b < 4; ++b) {
-                        const int r = 4 * rr + a, c = 4 * cc + b;
-                        if (rr >= 0 && r < mt && r >= c)
-                            A11[(c0 + IB + r) + (int64_t)(c0 + IB + c) * lda] = acc[u][a][b];
-                    }
+                for (int r = 0; r < 4; ++r) A11[row + (int64_t)(BT * p + Acc<T>::row(lane, r)) * lda] = -acc[s][r] * ns[r];
             }
         }
-        __syncthreads();
     }
 }
 
-// Column block cb (IB columns) of Linv for the factored nb x nb diagonal
-// block (lower triangle of A); the diagonal IB-blocks of Linv are already
-// stored.  Rows above the column block are zero.
-template <typename T>
+// Column block(s) cb of Linv, NT tiles of 16 columns a workgroup (1; 2 for
+// comparison runs, the same bits), for the factored nb x nb diagonal block
+// (lower triangle of A); the diagonal tiles of Linv are already stored.  Rows
+// above the diagonal tile are zero.
+template <typename T, int NT>
 __device__ __forceinline__ void diag_inverse_body(const T* __restrict__ A, int64_t lda, int nb, T* __restrict__ Linv,
                                                   int64_t ldl, int cb) {
-    __shared__ T Xs[FACT_NB][IB + 1];           // rows c0.. of the column block
-    __shared__ T Lr[IB][FACT_NB - IB + 1];      // L(r0 + i, c0 + q), q < r0 - c0
-    __shared__ T Mr[IB][IB + 1];                // Mi of block row r0
-    __shared__ T Tt[IB][IB + 1];
-    const int tid = threadIdx.x;
-    const int c0 = cb * IB;
-    if (c0 >= nb) return;
-    const int wc = min(IB, nb - c0);
-    for (int t = tid; t < c0 * wc; t += DIAG_THREADS) {
-        const int i = t % c0, j = t / c0;
-        Linv[i + (int64_t)(c0 + j) * ldl] = T(0);
-    }
-    for (int t = tid; t < IB * IB; t += DIAG_THREADS) {
-        const int i = t % IB, j = t / IB;
-        Xs[i][j] = (i < wc && j < wc) ? Linv[(c0 + i) + (int64_t)(c0 + j) * ldl] : T(0);
-    }
-    const int ti = tid / (IB / 2), tj = 2 * (tid % (IB / 2));   // 32 rows x 16 column pairs
-    for (int r0 = c0 + IB; r0 < nb; r0 += IB) {
-        const int rw = min(IB, nb - r0);
-        const int K = r0 - c0;
-        for (int t = tid; t < IB * K; t += DIAG_THREADS) {
-            const int i = t % IB, q = t / IB;
-            Lr[i][q] = (i < rw) ? A[(r0 + i) + (int64_t)(c0 + q) * lda] : T(0);
+    typedef typename Acc<T>::type acc_t;
+    __shared__ T xb[2][NT][4][64];         // X_q as a B operand, two steps
+    __builtin_amdgcn_s_setprio(3);
+    constexpr int NW = DIAG_THREADS / 64;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int li = lane & 15;
+    const int np = (nb + BT - 1) / BT, c = cb * NT;
+    if (c >= np) return;
+    auto at = [&](const T* p, int64_t ld, int row, int col) -> T {   // clamped, as in diag_body
+        return p[min(row, nb - 1) + (int64_t)min(col, nb - 1) * ld];
+    };
+    // -Mi of the wave's tile rows, the diagonal tiles of the column blocks,
+    // and L of the update of step q, one step ahead
+    T m[INV_SLOTS][4], xd[NT][4], l[INV_SLOTS][4];
+    auto load_l = [&](int q) {
+#pragma unroll
+        for (int s = 0; s < INV_SLOTS; ++s)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) l[s][k] = at(A, lda, BT * (wave + NW * s) + li, BT * q + Acc<T>::row(lane, k));
+    };
+    load_l(c);
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            xd[n][k] = at(Linv, ldl, BT * (c + n) + Acc<T>::row(lane, k), BT * (c + n) + li);
+#pragma unroll
+    for (int s = 0; s < INV_SLOTS; ++s)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            // (a factor, not a select, clears the columns beyond nb)
+            const int r = BT * (wave + NW * s), col = r + Acc<T>::row(lane, k);
+            m[s][k] = at(Linv, ldl, r + li, col) * (col < nb ? T(-1) : T(0));
         }
-        for (int t = tid; t < IB * IB; t += DIAG_THREADS) {
-            const int i = t % IB, j = t / IB;
-            Mr[i][j] = (i < rw && j < rw) ? Linv[(r0 + i) + (int64_t)(r0 + j) * ldl] : T(0);
-        }
-        __syncthreads();
-        {
-            T a0 = 0, a1 = 0;
-            for (int q = 0; q < K; ++q) {
-                const T l = Lr[ti][q];
-                a0 += l * Xs[q][tj];
-                a1 += l * Xs[q][tj + 1];
+    // zero rows above the diagonal tile of each column
+    for (int t = threadIdx.x; t < BT * NT * (c + NT) * BT; t += DIAG_THREADS) {
+        const int i = t % ((c + NT) * BT), j = c * BT + t / ((c + NT) * BT);
+        if (i < j / BT * BT && j < nb) Linv[i + (int64_t)j * ldl] = T(0);
+    }
+    acc_t acc[INV_SLOTS][NT];
+#pragma unroll
+    for (int s = 0; s < INV_SLOTS; ++s)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[s][n] = acc_t{0, 0, 0, 0};
+    for (int q = c; q < np; ++q) {
+        T (*x)[4][64] = xb[q & 1];
+        if (q % NW == wave) {
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+                acc_t v = {0, 0, 0, 0};
+                if (q > c + n) {
+#pragma unroll
+                    for (int s = 0; s < INV_SLOTS; ++s)
+                        if (wave + NW * s == q) {
+#pragma unroll
+                            for (int k = 0; k < 4; ++k) v = Acc<T>::mfma(m[s][k], acc[s][n][k], v);
+                        }
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const int row = BT * q + Acc<T>::row(lane, k), col = BT * (c + n) + li;
+                        if (row < nb && col < nb) Linv[row + (int64_t)col * ldl] = v[k];
+                    }
+                } else if (q == c + n) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) v[k] = xd[n][k];
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k) x[n][k][lane] = v[k];
             }
-            Tt[ti][tj] = a0;
-            Tt[ti][tj + 1] = a1;
         }
+        T lq[INV_SLOTS][4];
+#pragma unroll
+        for (int s = 0; s < INV_SLOTS; ++s)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) lq[s][k] = l[s][k];
+        if (q + 1 < np) load_l(q + 1);
         __syncthreads();
-        {
-            T a0 = 0, a1 = 0;
-            for (int l = 0; l <= ti; ++l) {
-                const T mm = Mr[ti][l];
-                a0 += mm * Tt[l][tj];
-                a1 += mm * Tt[l][tj + 1];
-            }
-            Xs[K + ti][tj] = -a0;
-            Xs[K + ti][tj + 1] = -a1;
-        }
-        __syncthreads();
-    }
-    const int rows = nb - c0 - IB;
-    for (int t = tid; t < rows * wc; t += DIAG_THREADS) {
-        const int i = t % rows, j = t / rows;
-        Linv[(c0 + IB + i) + (int64_t)(c0 + j) * ldl] = Xs[IB + i][j];
+#pragma unroll
+        for (int s = 0; s < INV_SLOTS; ++s)
+            if (wave + NW * s > q)
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+                    if (q >= c + n)
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) acc[s][n] = Acc<T>::mfma(lq[s][k], x[n][k][lane], acc[s][n]);
     }
 }
-
-// FP64 variant of diag_inverse_body with a third of the LDS (47.6 KB
-// against 142 KB), so that its workgroups start on a CU beside one running
-// FP64 trailing-update workgroup (73.7 KB) instead of waiting for an empty
-// CU: each workgroup builds 16 columns of Linv (the columns of a forward
-// substitution are independent), and the block row L(r0.., c0..r0) is staged
-// 32 columns at a time through a buffer that then holds Mi of the block row.
-// Every entry sums its products in the same order as diag_inverse_body, so
-// the two give the same bits.  Workgroup cb: columns 16 cb .. 16 cb + 15.
-constexpr int INV64_CW = 16;
-__device__ __forceinline__ void diag_inverse_body_f64(const double* __restrict__ A, int64_t lda, int nb,
-                                                      double* __restrict__ Linv, int64_t ldl, int cb) {
-    __shared__ double Xs[FACT_NB][INV64_CW + 1];   // rows c0.. of the columns j0 .. j0 + 15
-    __shared__ double Ls[IB][IB + 1];              // a 32-column chunk of the block row, then Mi of the row
-    __shared__ double Tt[IB][INV64_CW + 1];
-    const int tid = threadIdx.x;
-    const int j0 = cb * INV64_CW;
-    if (j0 >= nb) return;
-    const int c0 = j0 / IB * IB;                   // the IB-block the columns lie in
-    const int jo = j0 - c0;                        // their offset inside it
-    const int wc = min(INV64_CW, nb - j0);
-    for (int t = tid; t < c0 * wc; t += DIAG_THREADS) {
-        const int i = t % c0, j = t / c0;
-        Linv[i + (int64_t)(j0 + j) * ldl] = 0.0;
-    }
-    const int dw = min(IB, nb - c0);               // rows of the diagonal IB-block
-    for (int t = tid; t < IB * INV64_CW; t += DIAG_THREADS) {
-        const int i = t % IB, j = t / IB;
-        Xs[i][j] = (i < dw && j < wc) ? Linv[(c0 + i) + (int64_t)(j0 + j) * ldl] : 0.0;
-    }
-    const int ti = tid / INV64_CW, tj = tid % INV64_CW;   // 32 rows x 16 columns
-    for (int r0 = c0 + IB; r0 < nb; r0 += IB) {
-        const int rw = min(IB, nb - r0);
-        const int K = r0 - c0;
-        double a = 0.0;
-        for (int q0 = 0; q0 < K; q0 += IB) {
-            __syncthreads();                       // Xs rows written, the last chunk read
-            for (int t = tid; t < IB * IB; t += DIAG_THREADS) {
-                const int i = t % IB, q = t / IB;
-                Ls[i][q] = (i < rw) ? A[(r0 + i) + (int64_t)(c0 + q0 + q) * lda] : 0.0;
-            }
-            __syncthreads();
-            for (int q = 0; q < IB; ++q) a += Ls[ti][q] * Xs[q0 + q][tj];
-        }
-        Tt[ti][tj] = a;
-        __syncthreads();                           // Tt complete, Ls free
-        for (int t = tid; t < IB * IB; t += DIAG_THREADS) {
-            const int i = t % IB, j = t / IB;
-            Ls[i][j] = (i < rw && j < rw) ? Linv[(r0 + i) + (int64_t)(r0 + j) * ldl] : 0.0;
-        }
-        __syncthreads();
-        double b = 0.0;
-        for (int l = 0; l <= ti; ++l) b += Ls[ti][l] * Tt[l][tj];
-        Xs[K + ti][tj] = -b;
-    }
-    __syncthreads();
-    const int rows = nb - c0 - IB;
-    for (int t = tid; t < rows * wc; t += DIAG_THREADS) {
-        const int i = t % rows, j = t / rows;
-        Linv[(c0 + IB + i) + (int64_t)(j0 + j) * ldl] = Xs[IB + i][j];
-    }
-}
-
-// workgroups of the inverse of one diagonal block
-template <typename T>
-constexpr int inv_blocks() { return sizeof(T) == 8 ? FACT_NB / INV64_CW : FACT_NB / IB; }
 
 template <typename T>
 __global__ void __launch_bounds__(DF_THREADS) k_diag_factor(T* __restrict__ A, int64_t lda, int nb,
@@ -936,20 +998,10 @@ __global__ void __launch_bounds__(DF_THREADS) k_diag_factor(T* __restrict__ A, i
     diag_body<T>(A, lda, nb, sgn, info, k0, tiny, Linv, ldl);
 }
 
-template <typename T>
+template <typename T, int NT>
 __global__ void __launch_bounds__(DIAG_THREADS) k_diag_inverse(const T* __restrict__ A, int64_t lda, int nb,
                                                                T* __restrict__ Linv, int64_t ldl) {
-    if constexpr (sizeof(T) == 8)
-        diag_inverse_body_f64((const double*)A, lda, nb, (double*)Linv, ldl, blockIdx.x);
-    else
-        diag_inverse_body<T>(A, lda, nb, Linv, ldl, blockIdx.x);
-}
-
-// The 32-column FP64 inverse (142 KB of LDS), for comparison runs
-// (OMH_DIAG_INV64_WIDE=1).
-__global__ void __launch_bounds__(DIAG_THREADS) k_diag_inverse_wide64(const double* __restrict__ A, int64_t lda,
-                                                                      int nb, double* __restrict__ Linv, int64_t ldl) {
-    diag_inverse_body<double>(A, lda, nb, Linv, ldl, blockIdx.x);
+    diag_inverse_body<T, NT>(A, lda, nb, Linv, ldl, blockIdx.x);
 }
 
 // One workgroup per diagonal block of several factorisations.
@@ -963,10 +1015,7 @@ __global__ void __launch_bounds__(DF_THREADS) k_diag_grouped(const DiagDesc* __r
 template <typename T>
 __global__ void __launch_bounds__(DIAG_THREADS) k_diag_inverse_grouped(const DiagDesc* __restrict__ d) {
     const DiagDesc& g = d[blockIdx.y];
-    if constexpr (sizeof(T) == 8)
-        diag_inverse_body_f64((const double*)g.A11, g.lda, g.nb, (double*)g.Linv, FACT_NB, blockIdx.x);
-    else
-        diag_inverse_body<T>((const T*)g.A11, g.lda, g.nb, (T*)g.Linv, FACT_NB, blockIdx.x);
+    diag_inverse_body<T, 1>((const T*)g.A11, g.lda, g.nb, (T*)g.Linv, FACT_NB, blockIdx.x);
 }
 
 // Element-wise operations of several matrices (group = blockIdx.y).
@@ -2385,11 +2434,11 @@ void launch_grouped_diag(bool f32, const DiagDesc* d_descs, int ng, hipStream_t 
     if (f32) {
         k_diag_grouped<float><<<ng, DF_THREADS, 0, st>>>(d_descs, 1e-30f);
         OMH_LAUNCH_CHECK();
-        k_diag_inverse_grouped<float><<<dim3(inv_blocks<float>(), (unsigned)ng), DIAG_THREADS, 0, st>>>(d_descs);
+        k_diag_inverse_grouped<float><<<dim3(DF_TILES, (unsigned)ng), DIAG_THREADS, 0, st>>>(d_descs);
     } else {
         k_diag_grouped<double><<<ng, DF_THREADS, 0, st>>>(d_descs, 1e-290);
         OMH_LAUNCH_CHECK();
-        k_diag_inverse_grouped<double><<<dim3(inv_blocks<double>(), (unsigned)ng), DIAG_THREADS, 0, st>>>(d_descs);
+        k_diag_inverse_grouped<double><<<dim3(DF_TILES, (unsigned)ng), DIAG_THREADS, 0, st>>>(d_descs);
     }
     OMH_LAUNCH_CHECK();
 }
@@ -2606,13 +2655,12 @@ static void diag_factor(T* A, int64_t lda, int64_t k, int nb, T* Dinv, T* sgn, i
     ProfScope ps(sizeof(T) == 8 ? "diag_factor_f64" : "diag_factor_f32", (double)nb * nb * nb / 2.0, st);
     k_diag_factor<T><<<1, DF_THREADS, 0, st>>>(A11, lda, nb, sgn, info, k, tiny, Li, FACT_NB);
     OMH_LAUNCH_CHECK();
+    // 32 columns of the FP64 inverse per workgroup for comparison runs
     const char* wide64 = sizeof(T) == 8 ? std::getenv("OMH_DIAG_INV64_WIDE") : nullptr;
     if (wide64 && wide64[0] == '1')
-        k_diag_inverse_wide64<<<cdiv(nb, IB), DIAG_THREADS, 0, st>>>((const double*)A11, lda, nb, (double*)Li,
-                                                                     FACT_NB);
+        k_diag_inverse<T, 2><<<cdiv(nb, 2 * BT), DIAG_THREADS, 0, st>>>(A11, lda, nb, Li, FACT_NB);
     else
-        k_diag_inverse<T><<<cdiv(nb, sizeof(T) == 8 ? INV64_CW : IB), DIAG_THREADS, 0, st>>>(A11, lda, nb, Li,
-                                                                                          FACT_NB);
+        k_diag_inverse<T, 1><<<cdiv(nb, BT), DIAG_THREADS, 0, st>>>(A11, lda, nb, Li, FACT_NB);
     OMH_LAUNCH_CHECK();
 }
 
