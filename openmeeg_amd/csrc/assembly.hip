@@ -385,11 +385,15 @@ __global__ void __launch_bounds__(256, OMH_PAIR_MIN_WAVES) k_d_pairs(const TriRe
         const int np = c_nb_pts[order];
         for (int k = 0; k < np; ++k) {
             const double w = c_rules[order][k][3];
-            const d3 v = p1s_eval(o, gauss_point(order, k, P));
+            const d3 v = p1s_of(o, ana_eval(o, gauss_point(order, k, P)));
             rx += w * v.x;
             ry += w * v.y;
             rz += w * v.z;
         }
+        const d3 r = p1s_scale(o, mk(rx, ry, rz));
+        rx = r.x;
+        ry = r.y;
+        rz = r.z;
     }
     const double A = t1.area;
     W[(0 * n2 + j) * n1c + i] = A * rx;
@@ -631,38 +635,26 @@ __global__ void __launch_bounds__(256, OMH_PAIR_MIN_WAVES) k_pairs_fix(const Tri
         } else {
             constexpr int order = 3;
             const int np = c_nb_pts[order];
-            {   // S: OperatorS of t at the Gauss points of u
-                const OpS o = load_ops(T);
+            {   // S: OperatorS of t at the Gauss points of u, and from the
+                // same edge integrals D(u, t)
+                const AnaTri o = load_ana(T);
                 const d3 P[3] = {ld3(U.p[0]), ld3(U.p[1]), ld3(U.p[2])};
                 double res = 0.0;
-                for (int k = 0; k < np; ++k) res += c_rules[order][k][3] * ops_eval(o, gauss_point(order, k, P));
+                for (int k = 0; k < np; ++k) {
+                    const double wk = c_rules[order][k][3];
+                    const AnaVals v = ana_eval(o, gauss_point(order, k, P));
+                    res += wk * ops_of(o, v);
+                    if (DB) b = add(b, scl(wk, p1s_of(o, v)));
+                }
                 sv = (U.area * res) * ps.coeffS;
+                if (DB) b = (ps.diag && i == j) ? mk(0.0, 0.0, 0.0) : scl(U.area, p1s_scale(o, b));
             }
             if (DA) {   // D(t, u): P1 double layer of u at the Gauss points of t
-                const P1S o = load_p1s(U);
+                const AnaTri o = load_ana(U);
                 const d3 P[3] = {ld3(T.p[0]), ld3(T.p[1]), ld3(T.p[2])};
-                double rx = 0.0, ry = 0.0, rz = 0.0;
-                for (int k = 0; k < np; ++k) {
-                    const double wk = c_rules[order][k][3];
-                    const d3 v = p1s_eval(o, gauss_point(order, k, P));
-                    rx += wk * v.x;
-                    ry += wk * v.y;
-                    rz += wk * v.z;
-                }
-                a = mk(T.area * rx, T.area * ry, T.area * rz);
-            }
-            if (DB && !(ps.diag && i == j)) {   // D(u, t)
-                const P1S o = load_p1s(T);
-                const d3 P[3] = {ld3(U.p[0]), ld3(U.p[1]), ld3(U.p[2])};
-                double rx = 0.0, ry = 0.0, rz = 0.0;
-                for (int k = 0; k < np; ++k) {
-                    const double wk = c_rules[order][k][3];
-                    const d3 v = p1s_eval(o, gauss_point(order, k, P));
-                    rx += wk * v.x;
-                    ry += wk * v.y;
-                    rz += wk * v.z;
-                }
-                b = mk(U.area * rx, U.area * ry, U.area * rz);
+                for (int k = 0; k < np; ++k)
+                    a = add(a, scl(c_rules[order][k][3], p1s_of(o, ana_eval(o, gauss_point(order, k, P)))));
+                a = scl(T.area, p1s_scale(o, a));
             }
         }
         pair_store<DA, DB>(ps, H, L, i, il, j, sv, a, b);

@@ -108,79 +108,146 @@ __device__ __forceinline__ d3 gauss_point(int order, int i, const d3 P[3]) {
               b0 * P[0].z + b1 * P[1].z + b2 * P[2].z);
 }
 
-// Triangle "analytic side" of OperatorS, in registers.
-struct OpS {
+// ---------------------------------------------------------------------------
+// Analytic integrals over a triangle.  OperatorS and P1SingleLayerPotential
+// of one triangle at one point are both made of the three vertex distances
+// d_i, the edge integrals a_i = atanh(l_i / (d_i + d_{i+1})), the in-plane
+// edge offsets s_i = r_i.e_i, the height h and the solid angle; ana_eval
+// computes them once and ops_of / p1s_of combine them.  The P1 form uses
+//   log((d_{i+1} + r_{i+1}.U_i) / (d_i + r_i.U_i)) = 2 a_i   and
+//   (r_j x r_k).n = l s of the edge between j and k,
+// so it needs no logarithm, cross product or division of its own.
+// Bound by FP64 VALU issue.  Where every lane of a wave sees its triangle
+// from more than about 2.5 edge lengths (l/R < 0.2, |det/den| < 0.05) the
+// atanh and the arc tangent are short polynomials (relative errors 2.7e-17
+// and 3.4e-17); the other waves reduce the atanh's argument first and call
+// atan2 (a lane that satisfies the bounds gets the same bits either way, so
+// that a value does not depend on the lanes beside it).  Roots and reciprocals are the hardware estimates with one cubic
+// Newton step, within about an ulp.
+// ---------------------------------------------------------------------------
+struct AnaTri {            // triangle "analytic side", in registers
     d3 p0, p1, p2, n, e0, e1, e2;
-    double area, l0, l1, l2;
+    double l0, l1, l2, c01, c12, c02;   // edge lengths and the cosines U_i.U_j
+    double area2, inv_area;
 };
+typedef AnaTri OpS;
+typedef AnaTri P1S;
 
-__device__ __forceinline__ OpS load_ops(const TriRec& t) {
-    OpS o;
+__device__ __forceinline__ AnaTri load_ana(const TriRec& t) {
+    AnaTri o;
     o.p0 = ld3(t.p[0]); o.p1 = ld3(t.p[1]); o.p2 = ld3(t.p[2]);
     o.n = ld3(t.n);
     o.e0 = ld3(t.enrm[0]); o.e1 = ld3(t.enrm[1]); o.e2 = ld3(t.enrm[2]);
-    o.area = t.area;
     o.l0 = t.len[0]; o.l1 = t.len[1]; o.l2 = t.len[2];
-    return o;
-}
-
-// OperatorS::operator() (analytics.h:34-55) including the De Munck solid
-// angle of triangle.h:123-136.
-__device__ __forceinline__ double ops_eval(const OpS& o, d3 x) {
-    const d3 r0 = sub(o.p0, x), r1 = sub(o.p1, x), r2 = sub(o.p2, x);
-    const double d0 = norm(r0), d1 = norm(r1), d2 = norm(r2);
-    // atanh(l/R) written as log1p(2l/(R-l))/2: one division instead of two
-    double sum = dot(r0, o.e0) * (0.5 * log1p(2 * o.l0 / (d0 + d1 - o.l0)));
-    sum += dot(r1, o.e1) * (0.5 * log1p(2 * o.l1 / (d1 + d2 - o.l1)));
-    sum += dot(r2, o.e2) * (0.5 * log1p(2 * o.l2 / (d2 + d0 - o.l2)));
-    const double hn = dot(r0, o.n);
-    const double det = 2 * o.area * hn;
-    double omega = 0.0;
-    if (fabs(det) >= 1e-10) {
-        const double prod = d0 * d1 * d2;
-        const double den = prod + (d0 * dot(r1, r2) + d1 * dot(r2, r0) + d2 * dot(r0, r1));
-        omega = 2 * atan2(det, den);
-    }
-    return 2 * sum - hn * omega;
-}
-
-// Triangle "analytic side" of P1SingleLayerPotential, in registers.
-struct P1S {
-    d3 p0, p1, p2, n, U0, U1, U2;
-    double area, inv_area;
-};
-
-__device__ __forceinline__ P1S load_p1s(const TriRec& t) {
-    P1S o;
-    o.p0 = ld3(t.p[0]); o.p1 = ld3(t.p[1]); o.p2 = ld3(t.p[2]);
-    o.n = ld3(t.n);
-    o.U0 = ld3(t.U[0]); o.U1 = ld3(t.U[1]); o.U2 = ld3(t.U[2]);
-    o.area = t.area;
+    const d3 U0 = ld3(t.U[0]), U1 = ld3(t.U[1]), U2 = ld3(t.U[2]);
+    o.c01 = dot(U0, U1);
+    o.c12 = dot(U1, U2);
+    o.c02 = dot(U0, U2);
+    o.area2 = 2 * t.area;
     o.inv_area = t.inv_area;
     return o;
 }
+__device__ __forceinline__ OpS load_ops(const TriRec& t) { return load_ana(t); }
+__device__ __forceinline__ P1S load_p1s(const TriRec& t) { return load_ana(t); }
 
-// P1SingleLayerPotential::operator() (analytics.h:87-119).
-__device__ __forceinline__ d3 p1s_eval(const P1S& o, d3 x) {
-    const d3 r0 = sub(o.p0, x), r1 = sub(o.p1, x), r2 = sub(o.p2, x);
-    const double h = dot(r0, o.n);
-    if (fabs(h) < 1e-10) return mk(0.0, 0.0, 0.0);
-    const double d0 = norm(r0), d1 = norm(r1), d2 = norm(r2);
-    // S = sum_i U_i log((d_{i+1} + r_{i+1}.U_i) / (d_i + r_i.U_i))
-    const double g0 = log((d1 + dot(r1, o.U0)) / (d0 + dot(r0, o.U0)));
-    const double g1 = log((d2 + dot(r2, o.U1)) / (d1 + dot(r1, o.U1)));
-    const double g2 = log((d0 + dot(r0, o.U2)) / (d2 + dot(r2, o.U2)));
-    const d3 S = add(add(scl(g0, o.U0), scl(g1, o.U1)), scl(g2, o.U2));
-    const double dd = 2 * h * o.area;
-    const double d1v = d0 * d1 * d2 + (d0 * dot(r1, r2) + d1 * dot(r2, r0) + d2 * dot(r0, r1));
-    const double omega = atan2(dd, d1v);
-    const d3 D0 = sub(o.p1, o.p0), D1 = sub(o.p2, o.p1), D2 = sub(o.p0, o.p2);
-    const double E10 = dot(cross(r1, r2), o.n), E11 = dot(cross(r2, r0), o.n), E12 = dot(cross(r0, r1), o.n);
-    const double E20 = dot(D1, S), E21 = dot(D2, S), E22 = dot(D0, S);
-    const double hh = 0.5 * h;
-    return mk((omega * E10 + hh * E20) * o.inv_area, (omega * E11 + hh * E21) * o.inv_area,
-              (omega * E12 + hh * E22) * o.inv_area);
+__device__ __forceinline__ double rcp_fast(double x) {
+    const double y = __builtin_amdgcn_rcp(x);
+    const double e = fma(-x, y, 1.0);
+    return fma(y, fma(e, e, e), y);
 }
+__device__ __forceinline__ double sqrt_fast(double x) {   // finite x >= 0
+    const double y = __builtin_amdgcn_rsq(x);
+    const double g = x * y;
+    const double e = fma(-g, y, 1.0);
+    return x > 0.0 ? fma(g * e, fma(e, 0.375, 0.5), g) : x;
+}
+
+// atanh(z)/z for z^2 = u <= 0.04
+__device__ __forceinline__ double atanh_poly(double u) {
+    double p = fma(u, 0.07693501499136236, 0.07623676457223913);
+    p = fma(u, p, 0.09093263534125967);
+    p = fma(u, p, 0.11111066625651787);
+    p = fma(u, p, 0.1428571474076452);
+    p = fma(u, p, 0.19999999997718426);
+    p = fma(u, p, 0.33333333333337684);
+    return fma(u, p, 1.0);
+}
+
+// atanh(l/R), l < R: ((R+l)/(R-l)) = 2^k m with m in [1/sqrt2, sqrt2],
+// atanh(l/R) = k ln2/2 + atanh((m-1)/(m+1)); k = 0 and l/R itself below 0.2.
+__device__ __forceinline__ double atanh_edge(double l, double R) {
+    const double a = R + l, b = R - l;
+    const double ma = __builtin_amdgcn_frexp_mant(a);
+    double mb = __builtin_amdgcn_frexp_mant(b);
+    int k = __builtin_amdgcn_frexp_exp(a) - __builtin_amdgcn_frexp_exp(b);
+    const int up = (ma > 1.4142135623730951 * mb) - (ma < 0.7071067811865476 * mb);
+    mb = ldexp(mb, up);
+    const bool small = 5 * l < R;
+    const double num = small ? l : ma - mb, den = small ? R : ma + mb;
+    k = small ? 0 : k + up;
+    const double z = num * rcp_fast(den);
+    return fma((double)k, 0.34657359027997264, z * atanh_poly(z * z));
+}
+
+// atan(y/x) for |y/x| < 0.05
+__device__ __forceinline__ double atan_small(double y, double x) {
+    const double t = y * rcp_fast(x), u = t * t;
+    double p = fma(u, 0.11054487673653468, -0.1428559055751712);
+    p = fma(u, p, 0.19999999889582618);
+    p = fma(u, p, -0.33333333333298837);
+    return t * fma(u, p, 1.0);
+}
+
+struct AnaVals { double a0, a1, a2, s0, s1, s2, h, w; };   // w: half the solid angle
+
+__device__ __forceinline__ AnaVals ana_eval(const AnaTri& o, d3 x) {
+    AnaVals v;
+    const d3 r0 = sub(o.p0, x), r1 = sub(o.p1, x), r2 = sub(o.p2, x);
+    const double d0 = sqrt_fast(dot(r0, r0)), d1 = sqrt_fast(dot(r1, r1)), d2 = sqrt_fast(dot(r2, r2));
+    const double R0 = d0 + d1, R1 = d1 + d2, R2 = d2 + d0;
+    v.s0 = dot(r0, o.e0);
+    v.s1 = dot(r1, o.e1);
+    v.s2 = dot(r2, o.e2);
+    v.h = dot(r0, o.n);
+    const double det = o.area2 * v.h;
+    const double den = d0 * d1 * d2 + (d0 * dot(r1, r2) + d1 * dot(r2, r0) + d2 * dot(r0, r1));
+    const bool far = 5 * o.l0 < R0 && 5 * o.l1 < R1 && 5 * o.l2 < R2 && fabs(det) < 0.05 * den;
+    if (__ballot(!far) == 0) {
+        const double z0 = o.l0 * rcp_fast(R0), z1 = o.l1 * rcp_fast(R1), z2 = o.l2 * rcp_fast(R2);
+        v.a0 = z0 * atanh_poly(z0 * z0);
+        v.a1 = z1 * atanh_poly(z1 * z1);
+        v.a2 = z2 * atanh_poly(z2 * z2);
+        v.w = atan_small(det, den);
+    } else {
+        v.a0 = atanh_edge(o.l0, R0);
+        v.a1 = atanh_edge(o.l1, R1);
+        v.a2 = atanh_edge(o.l2, R2);
+        v.w = fabs(det) < 0.05 * den ? atan_small(det, den) : atan2(det, den);
+    }
+    return v;
+}
+
+// OperatorS::operator() (analytics.h:34-55) with the De Munck solid angle of
+// triangle.h:123-136.
+__device__ __forceinline__ double ops_of(const AnaTri& o, const AnaVals& v) {
+    const double hw = fabs(o.area2 * v.h) >= 1e-10 ? v.h * v.w : 0.0;
+    return 2 * (v.s0 * v.a0 + v.s1 * v.a1 + v.s2 * v.a2 - hw);
+}
+
+// P1SingleLayerPotential::operator() (analytics.h:87-119) without the factor
+// p1s_scale of each component, which is the same at every point.
+__device__ __forceinline__ d3 p1s_of(const AnaTri& o, const AnaVals& v) {
+    if (fabs(v.h) < 1e-10) return mk(0.0, 0.0, 0.0);
+    return mk(v.w * v.s1 + v.h * (o.c01 * v.a0 + v.a1 + o.c12 * v.a2),
+              v.w * v.s2 + v.h * (o.c02 * v.a0 + o.c12 * v.a1 + v.a2),
+              v.w * v.s0 + v.h * (v.a0 + o.c01 * v.a1 + o.c02 * v.a2));
+}
+__device__ __forceinline__ d3 p1s_scale(const AnaTri& o, d3 v) {
+    return mk(v.x * (o.inv_area * o.l1), v.y * (o.inv_area * o.l2), v.z * (o.inv_area * o.l0));
+}
+
+__device__ __forceinline__ double ops_eval(const OpS& o, d3 x) { return ops_of(o, ana_eval(o, x)); }
+__device__ __forceinline__ d3 p1s_eval(const P1S& o, d3 x) { return p1s_scale(o, p1s_of(o, ana_eval(o, x))); }
 
 // Dipole::potential (dipole.h:29-35); the 1/(4 pi) factor is applied outside.
 __device__ __forceinline__ double dip_potential(d3 r0, d3 q, d3 r) {
