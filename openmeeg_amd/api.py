@@ -578,8 +578,9 @@ class Factor:
     otherwise solve() raises NotConverged."""
 
     def __init__(self, L, n, work, precision, H64=None, structure=None, fallback_fp64=True, ipiv=None,
-                 n_positive=None, order=None):
+                 n_positive=None, order=None, ld=None):
         self.L, self.n, self.work, self.precision, self.H64 = L, n, work, precision, H64
+        self.ld = n if ld is None else ld   # leading dimension of L
         self.ipiv = ipiv
         self.iterations = 0
         self.rel_update = 0.0
@@ -603,7 +604,7 @@ class Factor:
         F = factor(H, self.n, "fp64", structure=self._raw_structure, n_positive=self.n_positive,
                    rebuild=(lambda: backup) if backup is not None else None)
         self.L, self.work, self.precision, self.H64, self.ipiv = F.L, F.work, F.precision, None, F.ipiv
-        self.order, self._fstructure = F.order, F._fstructure
+        self.order, self._fstructure, self.ld = F.order, F._fstructure, F.ld
         self.pivoted = F.pivoted
         self.fell_back = True
 
@@ -634,30 +635,30 @@ class Factor:
                 T = _dev_f64(self.n * nrhs)
                 check(lib().omh_reorder_rows_f64(_ptr(B), self.n, _ptr(T), self.n, self.n, nrhs, nseg, starts, optr,
                                                  0, _stream()))
-                check(lib().omh_sym_solve_f64_blocks(_ptr(self.L), self.n, self.n, _ptr(self.work), _ptr(T), self.n,
+                check(lib().omh_sym_solve_f64_blocks(_ptr(self.L), self.n, self.ld, _ptr(self.work), _ptr(T), self.n,
                                                      nrhs, *self._fstructure[2:], _stream()))
                 check(lib().omh_reorder_rows_f64(_ptr(T), self.n, _ptr(B), self.n, self.n, nrhs, nseg, starts, optr,
                                                  1, _stream()))
             elif blocks:
-                check(lib().omh_sym_solve_f64_blocks(_ptr(self.L), self.n, self.n, _ptr(self.work), _ptr(B), self.n,
+                check(lib().omh_sym_solve_f64_blocks(_ptr(self.L), self.n, self.ld, _ptr(self.work), _ptr(B), self.n,
                                                      nrhs, *blocks, _stream()))
             else:
-                check(lib().omh_sym_solve_f64(_ptr(self.L), self.n, self.n, _ptr(self.work), _ptr(B), self.n, nrhs,
+                check(lib().omh_sym_solve_f64(_ptr(self.L), self.n, self.ld, _ptr(self.work), _ptr(B), self.n, nrhs,
                                               _stream()))
             return B
         X = _dev_f64(self.n * nrhs)
         it, rel = C.c_int32(), C.c_double()
         if self.order is not None:
-            rc = lib().omh_mixed_solve_reordered(_ptr(self.H64), self.n, self.n, _ptr(self.L), self.n,
+            rc = lib().omh_mixed_solve_reordered(_ptr(self.H64), self.n, self.n, _ptr(self.L), self.ld,
                                                  _ptr(self.work), _ptr(B), self.n, _ptr(X), self.n, nrhs, max_iter,
                                                  tol, *blocks, self.order.ctypes.data_as(C.c_void_p), C.byref(it),
                                                  C.byref(rel), _stream())
         elif blocks:
-            rc = lib().omh_mixed_solve_blocks(_ptr(self.H64), self.n, self.n, _ptr(self.L), self.n, _ptr(self.work),
+            rc = lib().omh_mixed_solve_blocks(_ptr(self.H64), self.n, self.n, _ptr(self.L), self.ld, _ptr(self.work),
                                               _ptr(B), self.n, _ptr(X), self.n, nrhs, max_iter, tol, *blocks,
                                               C.byref(it), C.byref(rel), _stream())
         else:
-            rc = lib().omh_mixed_solve(_ptr(self.H64), self.n, self.n, _ptr(self.L), self.n, _ptr(self.work),
+            rc = lib().omh_mixed_solve(_ptr(self.H64), self.n, self.n, _ptr(self.L), self.ld, _ptr(self.work),
                                        _ptr(B), self.n, _ptr(X), self.n, nrhs, max_iter, tol, C.byref(it),
                                        C.byref(rel), _stream())
         self.iterations, self.rel_update = it.value, rel.value
@@ -776,20 +777,23 @@ def factor(Hdev, n, precision="fp64", structure=None, n_positive=None, rebuild=N
         F = Factor(L, n, work, "fp64", structure=structure, n_positive=n_positive, order=order)
         elem = 8
     elif precision in ("mixed", "mixed16"):
-        L32 = torch.empty(n * n, dtype=torch.float32, device="cuda")
+        # the reordered copy's columns start on 16 bytes: vector loads in the
+        # panels, and the split products of the solves
+        ld = n if order is None else (n + 3) // 4 * 4
+        L32 = torch.empty(ld * n, dtype=torch.float32, device="cuda")
         if order is not None:
-            check(lib().omh_sym_reorder(_ptr(Hdev), n, _ptr(L32), n, 4, n, blocks[0], blocks[1], optr, _stream()))
+            check(lib().omh_sym_reorder(_ptr(Hdev), n, _ptr(L32), ld, 4, n, blocks[0], blocks[1], optr, _stream()))
         else:
             check(lib().omh_convert_f64_f32(_ptr(Hdev), n, _ptr(L32), n, n, n, 1, _stream()))
         work = torch.empty(int(lib().omh_factor_workspace_bytes(n, 4)), dtype=torch.uint8, device="cuda")
         if blocks:
             fn = lib().omh_sym_factor_f32_blocks if precision == "mixed" else lib().omh_sym_factor_f32_split_blocks
-            check(fn(_ptr(L32), n, n, _ptr(work), *(fblocks if order is not None else blocks), C.byref(info),
+            check(fn(_ptr(L32), n, ld, _ptr(work), *(fblocks if order is not None else blocks), C.byref(info),
                      _stream()))
         else:
             fn = lib().omh_sym_factor_f32 if precision == "mixed" else lib().omh_sym_factor_f32_split
             check(fn(_ptr(L32), n, n, _ptr(work), C.byref(info), _stream()))
-        F = Factor(L32, n, work, "mixed", H64=Hdev, structure=structure, n_positive=n_positive, order=order)
+        F = Factor(L32, n, work, "mixed", H64=Hdev, structure=structure, n_positive=n_positive, order=order, ld=ld)
         elem = 4
     else:
         raise ValueError("precision must be 'fp64', 'mixed', 'mixed16' or 'fp64_lu'")

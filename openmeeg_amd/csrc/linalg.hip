@@ -82,6 +82,10 @@ template <typename T> struct Vec;
 template <> struct Vec<float> { typedef float4 type; static constexpr int n = 4; };
 template <> struct Vec<double> { typedef double2 type; static constexpr int n = 2; };
 
+// k-slices a 64 x 64 tile keeps in flight in registers (more of FP64 would
+// leave two waves on a SIMD instead of three).
+template <typename T> struct InFlight { static constexpr int v = sizeof(T) == 4 ? 4 : 2; };
+
 // Loads an R x BK operand tile into registers.  MK: element (r, kk) at
 // base[r + kk*ld] (contiguous along r); else base[kk + r*ld] (contiguous
 // along kk).  load_full: the tile is in range and 16-byte aligned (vector
@@ -121,6 +125,23 @@ struct TileLoader {
             for (int q = 0; q < V; ++q) {
                 const int64_t rr = r0 + r + (MK ? q : 0), kq = k0 + kk + (MK ? 0 : q);
                 reg[p][q] = (rr < rmax && kq < kmax) ? (MK ? base[rr + kq * ld] : base[kq + rr * ld]) : T(0);
+            }
+        }
+    }
+
+    // Rows past rmax read row rmax - 1 (they reach no stored entry), k in
+    // range: element-wise loads that nothing selects on (a guard around each
+    // one becomes a branch that waits for it).
+    __device__ __forceinline__ void load_clamped(const T* __restrict__ base, int64_t ld, int64_t r0, int64_t k0,
+                                                 int64_t rmax, int tid) {
+#pragma unroll
+        for (int p = 0; p < NV; ++p) {
+            int r, kk;
+            coords(tid + 256 * p, r, kk);
+#pragma unroll
+            for (int q = 0; q < V; ++q) {
+                const int64_t rr = min(r0 + r + (MK ? q : 0), rmax - 1), kq = k0 + kk + (MK ? 0 : q);
+                reg[p][q] = MK ? base[rr + kq * ld] : base[kq + rr * ld];
             }
         }
     }
@@ -250,8 +271,12 @@ __device__ __forceinline__ void gemm_tile(int64_t m, int64_t n, int64_t k, T alp
 #pragma unroll
         for (int b = 0; b < WB; ++b) acc[a][b] = typename Acc<T>::type{0, 0, 0, 0};
 
-    TileLoader<T, !TA, BM> la;
-    TileLoader<T, TB, BN> lb;
+    // PF slices in flight in registers: a workgroup of 64 x 64 tiles is often
+    // alone on its CU, and one slice ahead left it waiting for memory (1.1 us
+    // a slice)
+    constexpr int PF = WB == 2 ? InFlight<T>::v : 1;
+    TileLoader<T, !TA, BM> la[PF];
+    TileLoader<T, TB, BN> lb[PF];
 
     auto compute = [&](const T* Ab, const T* Bb) {
 #pragma unroll
@@ -269,59 +294,47 @@ __device__ __forceinline__ void gemm_tile(int64_t m, int64_t n, int64_t k, T alp
         }
     };
 
-    if (!EDGE) {
-        const int64_t nk = k / BK;   // full k-slices
-        if (nk > 0) {
-            la.load_full(A, lda, row0, 0, tid);
-            lb.load_full(B, ldb, col0, 0, tid);
-            la.store(As[0], tid);
-            lb.store(Bs[0], tid);
-            __syncthreads();
-            for (int64_t kt = 0; kt < nk; ++kt) {
-                const int buf = (int)(kt & 1);
-                if (kt + 1 < nk) {
-                    la.load_full(A, lda, row0, (kt + 1) * BK, tid);
-                    lb.load_full(B, ldb, col0, (kt + 1) * BK, tid);
-                }
+    const int64_t nk = k / BK;   // full k-slices
+    // slice sl into ring slot u (past the end: the last slice again, unused)
+    auto load = [&](int u, int64_t sl) {
+        const int64_t k0 = min(sl, nk - 1) * BK;
+        if (EDGE) {
+            la[u].load_clamped(A, lda, row0, k0, m, tid);
+            lb[u].load_clamped(B, ldb, col0, k0, n, tid);
+        } else {
+            la[u].load_full(A, lda, row0, k0, tid);
+            lb[u].load_full(B, ldb, col0, k0, tid);
+        }
+    };
+    if (nk > 0) {
+#pragma unroll
+        for (int u = 0; u < PF; ++u) load(u, u);
+        la[0].store(As[0], tid);
+        lb[0].store(Bs[0], tid);
+        load(0, PF);
+        __syncthreads();
+        for (int64_t kt0 = 0; kt0 < nk; kt0 += PF) {
+#pragma unroll
+            for (int u = 0; u < PF; ++u) {
+                const int64_t kt = kt0 + u;
+                if (kt >= nk) break;
+                constexpr bool even = PF % 2 == 0;
+                const int buf = even ? (u & 1) : (int)(kt & 1), nx = (u + 1) % PF;
+                la[nx].store(As[buf ^ 1], tid);
+                lb[nx].store(Bs[buf ^ 1], tid);
+                load(nx, kt + 1 + PF);
                 compute(As[buf], Bs[buf]);
-                if (kt + 1 < nk) {
-                    la.store(As[buf ^ 1], tid);
-                    lb.store(Bs[buf ^ 1], tid);
-                }
                 __syncthreads();
             }
         }
-        if (k % BK) {   // partial last k-slice
-            la.load_guarded(A, lda, row0, nk * BK, m, k, tid);
-            lb.load_guarded(B, ldb, col0, nk * BK, n, k, tid);
-            la.store(As[0], tid);
-            lb.store(Bs[0], tid);
-            __syncthreads();
-            compute(As[0], Bs[0]);
-        }
-    } else {
-        // the same double-buffered pipeline with guarded loads
-        const int64_t nk = (k + BK - 1) / BK;
-        if (nk > 0) {
-            la.load_guarded(A, lda, row0, 0, m, k, tid);
-            lb.load_guarded(B, ldb, col0, 0, n, k, tid);
-            la.store(As[0], tid);
-            lb.store(Bs[0], tid);
-            __syncthreads();
-            for (int64_t kt = 0; kt < nk; ++kt) {
-                const int buf = (int)(kt & 1);
-                if (kt + 1 < nk) {
-                    la.load_guarded(A, lda, row0, (kt + 1) * BK, m, k, tid);
-                    lb.load_guarded(B, ldb, col0, (kt + 1) * BK, n, k, tid);
-                }
-                compute(As[buf], Bs[buf]);
-                if (kt + 1 < nk) {
-                    la.store(As[buf ^ 1], tid);
-                    lb.store(Bs[buf ^ 1], tid);
-                }
-                __syncthreads();
-            }
-        }
+    }
+    if (k % BK) {   // partial last k-slice
+        la[0].load_guarded(A, lda, row0, nk * BK, m, k, tid);
+        lb[0].load_guarded(B, ldb, col0, nk * BK, n, k, tid);
+        la[0].store(As[0], tid);
+        lb[0].store(Bs[0], tid);
+        __syncthreads();
+        compute(As[0], Bs[0]);
     }
     // Epilogue.  FP32: a lane's 4 elements are 4 consecutive rows of one
     // column, written with one 16-byte access on interior tiles.
@@ -3677,8 +3690,18 @@ static void sym_solve_impl(const T* L, int64_t n, int64_t lda, const void* work,
     constexpr int64_t GW = (int64_t)SOLVE_GROUP * FACT_NB;
     std::vector<std::pair<int64_t, int64_t>> iv;
     // The split products need 16-byte aligned columns of L (backward) and
-    // serve the full groups; the others take the FP32 products.
+    // serve the full groups whose product fills the chip with their 128 x 256
+    // tiles; the others take the FP32 products.
     const bool split_ok = sb && sizeof(T) == 4 && lda % 4 == 0 && reinterpret_cast<uintptr_t>(L) % 16 == 0;
+    // Four 64 x 64 FP32 tiles a CU is where the two meet: at 128 right-hand
+    // sides over up to 15000 rows the split products take 60 us a group (half
+    // of each tile is padding) and the FP32 ones about 45, at 256 over
+    // 30000 rows 120 us and about 130.
+    auto fills = [&](const std::vector<std::pair<int64_t, int64_t>>& v) {
+        int64_t rows = 0;
+        for (const auto& x : v) rows += x.second - x.first;
+        return cdiv(rows, 64) * cdiv(r, 64) >= 1024;
+    };
     // strips of 2 right-hand sides up to 1024 of them (128 workgroups for
     // 256; 8-wide strips took twice as long per group at 256), else 8
     const bool narrow = r <= 1024;
@@ -3719,16 +3742,16 @@ static void sym_solve_impl(const T* L, int64_t n, int64_t lda, const void* work,
         OMH_HIP(hipStreamWaitEvent(la->side, la->ready, 0));
         for (int64_t k0 = 0, gi = 0; k0 < n; k0 += GW, ++gi) {
             const int64_t gend = std::min<int64_t>(k0 + GW, n);
-            if (gend - k0 == GW && gend < n) {
-                rows_below(k0, gend);
+            if (gend - k0 == GW && gend < n) rows_below(k0, gend);
+            if (gend - k0 == GW && gend < n && fills(iv)) {
                 form_scales(false, (const float*)L, lda, k0, iv, scale_slot(false, k0, *sb), la->side);
             }
             if ((gi + 1) % chunk == 0 || gend >= n) OMH_HIP(hipEventRecord(la->scale_ev[gi / chunk], la->side));
         }
         for (int64_t k0 = ((n - 1) / GW) * GW, bi = 0; k0 >= 0; k0 -= GW, ++bi) {
             const int64_t gend = std::min<int64_t>(k0 + GW, n);
-            if (gend - k0 == GW && k0 > 0) {
-                cols_before(k0, gend);
+            if (gend - k0 == GW && k0 > 0) cols_before(k0, gend);
+            if (gend - k0 == GW && k0 > 0 && fills(iv)) {
                 form_scales(true, (const float*)L, lda, k0, iv, scale_slot(true, k0, *sb), la->side);
             }
             if ((bi + 1) % chunk == 0 || k0 == 0)
@@ -3738,10 +3761,10 @@ static void sym_solve_impl(const T* L, int64_t n, int64_t lda, const void* work,
     // forward: W <- L^-1 W
     for (int64_t k0 = 0, gi = 0; k0 < n; k0 += GW, ++gi) {
         const int64_t gend = std::min<int64_t>(k0 + GW, n);
-        const bool split = split_ok && gend - k0 == GW && gend < n;
+        if (gend < n) rows_below(k0, gend);
+        const bool split = split_ok && gend - k0 == GW && gend < n && fills(iv);
         group_solve(false, k0, gend, split);
         if (gend < n) {
-            rows_below(k0, gend);
             if (split)
                 split_solve_update(false, (const float*)L, lda, k0, iv, *sb, (float*)W, ldw, r, st,
                                    ahead ? la->scale_ev[gi / chunk] : nullptr);
@@ -3758,11 +3781,11 @@ static void sym_solve_impl(const T* L, int64_t n, int64_t lda, const void* work,
     // groups' contributions)
     for (int64_t k0 = ((n - 1) / GW) * GW, bi = 0; k0 >= 0; k0 -= GW, ++bi) {
         const int64_t gend = std::min<int64_t>(k0 + GW, n);
-        const bool split = split_ok && gend - k0 == GW && k0 > 0;
+        if (k0 > 0) cols_before(k0, gend);
+        const bool split = split_ok && gend - k0 == GW && k0 > 0 && fills(iv);
         group_solve(true, k0, gend, split);
         // rows above the group: only the columns its rows reach in L
         if (k0 > 0) {
-            cols_before(k0, gend);
             if (split)
                 split_solve_update(true, (const float*)L, lda, k0, iv, *sb, (float*)W, ldw, r, st,
                                    ahead ? la->scale_ev[SCALE_EVENTS / 2 + bi / chunk] : nullptr);
@@ -3997,7 +4020,8 @@ int mixed_refine(const double* H, int64_t n, int64_t ldh, const float* L32, int6
                  double* final_rel_update, bool* converged, hipStream_t st, const BlockFill* bf,
                  const FactorOrder* fo) {
     RefineBuffers buf;
-    buf.R32 = (float*)scratch(SCR_LINALG, sizeof(float) * (size_t)n * (size_t)r, st);
+    buf.ldr32 = (n + 3) / 4 * 4;   // 16-byte aligned columns: the solves' vector loads
+    buf.R32 = (float*)scratch(SCR_LINALG, sizeof(float) * (size_t)buf.ldr32 * (size_t)r, st);
     buf.R = (double*)scratch(SCR_ASSEMBLY, sizeof(double) * (size_t)n * (size_t)r, st);
     buf.part = (double*)scratch(SCR_SMALL, sizeof(double) * NORM_PARTS, st);
     buf.split = scratch(SCR_LINALG2, split_solve_bytes(n, r), st);
@@ -4017,6 +4041,7 @@ int mixed_refine_in(const double* H, int64_t n, int64_t ldh, const float* L32, i
     const BlockFill* bfl = fo ? &fo->fill : bf;
     const int32_t* rowmap = fo ? fo->rowmap : nullptr;
     float* R32 = buf.R32;
+    const int64_t ldq = buf.ldr32 ? buf.ldr32 : n;
     double* R = buf.R;
     SplitSolveBuf sb;
     if (buf.split) {
@@ -4034,14 +4059,14 @@ int mixed_refine_in(const double* H, int64_t n, int64_t ldh, const float* L32, i
     RefineState state = REFINE_CONTINUE;
     for (; it < max_iter; ++it) {
         if (rowmap) {
-            k_rows_map<double, float><<<grid_for(n * r), 256, 0, st>>>(R, n, R32, n, n, r, rowmap, 0);
+            k_rows_map<double, float><<<grid_for(n * r), 256, 0, st>>>(R, n, R32, ldq, n, r, rowmap, 0);
             OMH_LAUNCH_CHECK();
         } else {
-            convert_f64_to_f32(R, n, R32, n, n, r, false, st);
+            convert_f64_to_f32(R, n, R32, ldq, n, r, false, st);
         }
-        sym_solve_impl<float>(L32, n, ld32, work32, R32, n, r, st, bfl, buf.split ? &sb : nullptr);
+        sym_solve_impl<float>(L32, n, ld32, work32, R32, ldq, r, st, bfl, buf.split ? &sb : nullptr);
         sb.cached = sb.cache != nullptr;   // the same factor and structure on the next pass
-        k_axpy_f32_to_f64<<<grid_for(n * r), 256, 0, st>>>(R32, n, X, ldx, n, r, rowmap);
+        k_axpy_f32_to_f64<<<grid_for(n * r), 256, 0, st>>>(R32, ldq, X, ldx, n, r, rowmap);
         OMH_LAUNCH_CHECK();
         if (it == 0) {
             // X was zero, so the first update is X itself (relative size 1):
@@ -4049,7 +4074,7 @@ int mixed_refine_in(const double* H, int64_t n, int64_t ldh, const float* L32, i
             // all-zero right-hand side converges on the next pass instead)
             rel = 1.0;
         } else {
-            const double dn = frob_norm_with<float>(R32, n, n, r, buf.part, st);
+            const double dn = frob_norm_with<float>(R32, ldq, n, r, buf.part, st);
             const double xn = frob_norm_with<double>(X, ldx, n, r, buf.part, st);
             rel = xn > 0 ? dn / xn : (dn > 0 ? 1.0 : 0.0);
         }

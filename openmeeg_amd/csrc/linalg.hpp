@@ -284,6 +284,7 @@ int mixed_refine(const double* H, int64_t n, int64_t ldh, const float* L32, int6
 constexpr int NORM_PARTS = 1024;
 struct RefineBuffers {
     float* R32 = nullptr;
+    int64_t ldr32 = 0;       // leading dimension of R32 (0: n)
     double* R = nullptr;
     double* part = nullptr;
     // optional: buffers of the split-FP16 products of the FP32 triangular
