@@ -249,17 +249,20 @@ __device__ __forceinline__ int64_t remap_tile(const TileRemap& r, int64_t x) {
 // TA: op(A)(i,kk) = A[kk + i*lda] (A stored k x m); else A[i + kk*lda].
 // TB: op(B)(kk,j) = B[j + kk*ldb] (B stored n x k); else B[kk + j*ldb].
 // LOWER: only entries with row >= col are written (m == n).
-// EDGE = false: every tile of the launch lies inside m x n and the operands
-// are 16-byte aligned, so the k loop uses unguarded vector loads (a partial
-// last k-slice is done after the loop).  EDGE = true: guarded loads.
+// EDGE = false: the tile lies inside m x n and the operands are 16-byte
+// aligned, so the k loop uses vector loads; EDGE = true: element loads with
+// clamped rows.  A partial last k-slice is done after the loop.  smem:
+// gemm_lds<T, WB>() elements of LDS.
+template <typename T, int WB> constexpr int gemm_lds() { return 4 * KSlice<T>::v * (32 * WB + LDS_PAD); }
 template <typename T, bool TA, bool TB, bool LOWER, int WB, bool EDGE>
 __device__ __forceinline__ void gemm_tile(int64_t m, int64_t n, int64_t k, T alpha, const T* __restrict__ A,
                                           int64_t lda, const T* __restrict__ B, int64_t ldb, T beta,
-                                          T* __restrict__ C, int64_t ldc, int64_t tm, int64_t tn) {
+                                          T* __restrict__ C, int64_t ldc, int64_t tm, int64_t tn, T* smem) {
     constexpr int BM = 32 * WB, BN = 32 * WB;
     constexpr int BK = KSlice<T>::v;
-    __shared__ T As[2][BK * (BM + LDS_PAD)];
-    __shared__ T Bs[2][BK * (BN + LDS_PAD)];
+    static_assert(BM == BN, "one slice size for both operands");
+    T (*As)[BK * (BM + LDS_PAD)] = reinterpret_cast<T (*)[BK * (BM + LDS_PAD)]>(smem);
+    T (*Bs)[BK * (BN + LDS_PAD)] = As + 2;
     const int64_t row0 = tm * BM, col0 = tn * BN;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
@@ -369,10 +372,27 @@ __device__ __forceinline__ void gemm_tile(int64_t m, int64_t n, int64_t k, T alp
         }
 }
 
-template <typename T, bool TA, bool TB, bool LOWER, int WB, bool EDGE>
+// One tile of a launch over all of C: the tiles inside m x n take the vector
+// loads, the partial last row and column of tiles the clamped ones, side by
+// side (as launches of their own the few workgroups of an edge strip took as
+// long as the interior: 36 us beside 42 us over 128 right-hand sides).
+// VEC = false (operands off 16 bytes): the clamped loads everywhere.
+template <typename T, bool TA, bool TB, bool LOWER, int WB, bool VEC>
+__device__ __forceinline__ void gemm_any_tile(int64_t m, int64_t n, int64_t k, T alpha, const T* __restrict__ A,
+                                              int64_t lda, const T* __restrict__ B, int64_t ldb, T beta,
+                                              T* __restrict__ C, int64_t ldc, int64_t tm, int64_t tn, T* smem) {
+    constexpr int TILE = 32 * WB;
+    if (VEC && (tm + 1) * TILE <= m && (tn + 1) * TILE <= n)
+        gemm_tile<T, TA, TB, LOWER, WB, false>(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, tm, tn, smem);
+    else
+        gemm_tile<T, TA, TB, LOWER, WB, true>(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, tm, tn, smem);
+}
+
+template <typename T, bool TA, bool TB, bool LOWER, int WB, bool VEC>
 __global__ void __launch_bounds__(256) k_gemm(int64_t m, int64_t n, int64_t k, T alpha, const T* __restrict__ A,
                                               int64_t lda, const T* __restrict__ B, int64_t ldb, T beta,
                                               T* __restrict__ C, int64_t ldc, TileMap map) {
+    __shared__ __align__(16) T smem[gemm_lds<T, WB>()];
     int64_t t = blockIdx.x;
     if (map.kind >= 4) {
         t = xcd_tile(t, map.per);
@@ -380,7 +400,7 @@ __global__ void __launch_bounds__(256) k_gemm(int64_t m, int64_t n, int64_t k, T
     }
     int64_t tm, tn;
     map_tile(map, t, tm, tn);
-    gemm_tile<T, TA, TB, LOWER, WB, EDGE>(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, tm, tn);
+    gemm_any_tile<T, TA, TB, LOWER, WB, VEC>(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, tm, tn, smem);
 }
 
 // Split-K product for outputs of few tiles with a long inner dimension:
@@ -388,16 +408,17 @@ __global__ void __launch_bounds__(256) k_gemm(int64_t m, int64_t n, int64_t k, T
 // y-th chunk of kc inner indices (the last one shorter), W_y at W + y m n
 // with leading dimension m.  k_splitk_sum then forms C = alpha sum_y W_y +
 // beta C, summing the chunks in order (deterministic).
-template <typename T, bool TA, bool TB, int WB, bool EDGE>
+template <typename T, bool TA, bool TB, int WB, bool VEC>
 __global__ void __launch_bounds__(256) k_gemm_splitk(int64_t m, int64_t n, int64_t k, int64_t kc,
                                                      const T* __restrict__ A, int64_t lda, const T* __restrict__ B,
                                                      int64_t ldb, T* __restrict__ W, TileMap map) {
+    __shared__ __align__(16) T smem[gemm_lds<T, WB>()];
     int64_t tm, tn;
     map_tile(map, blockIdx.x, tm, tn);
     const int64_t k0 = (int64_t)blockIdx.y * kc;
     const int64_t ks = k - k0 < kc ? k - k0 : kc;
-    gemm_tile<T, TA, TB, false, WB, EDGE>(m, n, ks, T(1), A + (TA ? k0 : k0 * lda), lda, B + (TB ? k0 * ldb : k0),
-                                          ldb, T(0), W + (int64_t)blockIdx.y * m * n, m, tm, tn);
+    gemm_any_tile<T, TA, TB, false, WB, VEC>(m, n, ks, T(1), A + (TA ? k0 : k0 * lda), lda, B + (TB ? k0 * ldb : k0),
+                                             ldb, T(0), W + (int64_t)blockIdx.y * m * n, m, tm, tn, smem);
 }
 
 template <typename T>
@@ -553,8 +574,9 @@ __global__ void __launch_bounds__(512) k_gemm_f64_dma(int64_t k, double alpha, c
 // Grouped GEMM: the tiles of ng independent products (descriptor d[g], its
 // tiles numbered from d[g].tile0) in one launch; each workgroup walks the
 // tile list with stride gridDim.x (persistent when the grid is capped).
-template <typename T, bool TA, bool TB, bool LOWER, int WB, bool EDGE>
+template <typename T, bool TA, bool TB, bool LOWER, int WB, bool VEC>
 __global__ void __launch_bounds__(256) k_gemm_grouped(const GemmDesc* __restrict__ d, int ng, int64_t total) {
+    __shared__ __align__(16) T smem[gemm_lds<T, WB>()];
     for (int64_t t = blockIdx.x; t < total; t += gridDim.x) {
         int lo = 0, hi = ng - 1;
         while (lo < hi) {
@@ -566,8 +588,8 @@ __global__ void __launch_bounds__(256) k_gemm_grouped(const GemmDesc* __restrict
         int64_t tm, tn;
         map_tile(g.map, t - g.tile0, tm, tn);
         __syncthreads();   // the previous tile's LDS reads are done
-        gemm_tile<T, TA, TB, LOWER, WB, EDGE>(g.m, g.n, g.k, (T)g.alpha, (const T*)g.A, g.lda, (const T*)g.B, g.ldb,
-                                              (T)g.beta, (T*)g.C, g.ldc, tm, tn);
+        gemm_any_tile<T, TA, TB, LOWER, WB, VEC>(g.m, g.n, g.k, (T)g.alpha, (const T*)g.A, g.lda, (const T*)g.B,
+                                                 g.ldb, (T)g.beta, (T*)g.C, g.ldc, tm, tn, smem);
     }
 }
 
@@ -2249,7 +2271,7 @@ inline unsigned grid_for(int64_t total) { return (unsigned)std::max<int64_t>(1, 
 // ---------------------------------------------------------------------------
 // host API
 // ---------------------------------------------------------------------------
-template <typename T, int WB, bool EDGE>
+template <typename T, int WB, bool VEC>
 static void launch_tiles(bool ta, bool tb, bool lower, int64_t nblk, TileMap map, int64_t m, int64_t n, int64_t k,
                          T alpha, const T* A, int64_t lda, const T* B, int64_t ldb, T beta, T* C, int64_t ldc,
                          hipStream_t st) {
@@ -2258,7 +2280,7 @@ static void launch_tiles(bool ta, bool tb, bool lower, int64_t nblk, TileMap map
     if (nblk > 0xffffffffLL) throw std::invalid_argument("gemm grid too large");
 #define OMH_GEMM_CASE(TA_, TB_, LO_)                                                                          \
     if (ta == TA_ && tb == TB_ && lower == LO_) {                                                             \
-        k_gemm<T, TA_, TB_, LO_, WB, EDGE><<<(unsigned)nblk, 256, 0, st>>>(m, n, k, alpha, A, lda, B, ldb, beta, \
+        k_gemm<T, TA_, TB_, LO_, WB, VEC><<<(unsigned)nblk, 256, 0, st>>>(m, n, k, alpha, A, lda, B, ldb, beta, \
                                                                            C, ldc, map);                      \
         OMH_LAUNCH_CHECK();                                                                                   \
         return;                                                                                               \
@@ -2272,7 +2294,7 @@ static void launch_tiles(bool ta, bool tb, bool lower, int64_t nblk, TileMap map
     throw std::invalid_argument("unsupported gemm variant");
 }
 
-// Tile map of an interior launch: the L2-aware order (kinds 4/5) when the
+// Tile map of a launch: the L2-aware order (kinds 4/5) when the
 // launch has enough tiles to spread over the XCDs, else the plain order.
 static TileMap l2_map(bool lower, int64_t fm, int64_t fn) {
     const int64_t tiles = lower ? fm * (fm + 1) / 2 : fm * fn;
@@ -2281,47 +2303,26 @@ static TileMap l2_map(bool lower, int64_t fm, int64_t fn) {
     return lower ? TileMap{4, fm, 0, 0, tiles, per} : TileMap{5, fm, 0, fn, tiles, per};
 }
 
-// Interior tiles run the unguarded kernel; the partial last tile row and
-// column (if any) run as edge strips.
+// All tiles of C in one launch.
 template <typename T, int WB>
 static void gemm_launch(bool ta, bool tb, bool lower, bool vec, int64_t m, int64_t n, int64_t k, T alpha, const T* A,
                         int64_t lda, const T* B, int64_t ldb, T beta, T* C, int64_t ldc, hipStream_t st,
                         const char* prof) {
     constexpr int TILE = 32 * WB;
     const int64_t ntm = cdiv(m, TILE), ntn = cdiv(n, TILE);
-    if (!vec) {
-        const int64_t nblk = lower ? ntm * (ntm + 1) / 2 : ntm * ntn;
-        launch_tiles<T, WB, true>(ta, tb, lower, nblk, TileMap{lower ? 1 : 0, ntm, 0, 0}, m, n, k, alpha, A, lda, B,
-                                  ldb, beta, C, ldc, st);
-        return;
-    }
-    const int64_t fm = m / TILE, fn = n / TILE;   // full tile rows / columns
-    if (lower) {
-        {
-            // optional timing of the interior launch; algorithmic work: the
-            // lower triangle of the interior square, (fm T)(fm T + 1) k flop
-            std::string name;
-            if (prof) name = std::string(prof) + "_t" + std::to_string(TILE);
-            const double side = (double)(fm * TILE);
-            ProfScope ps(prof ? name.c_str() : "", prof ? side * (side + 1) * (double)k : 0.0,
-                         prof ? st : nullptr);
-            if (!prof) ps.cancel();
-            launch_tiles<T, WB, false>(ta, tb, true, 0, l2_map(true, fm, fm), m, n, k, alpha, A, lda, B, ldb, beta,
-                                       C, ldc, st);
-        }
-        if (fm < ntm)   // last (partial) tile row, all its lower tiles
-            launch_tiles<T, WB, true>(ta, tb, true, ntm, TileMap{2, ntm, fm, 0}, m, n, k, alpha, A, lda, B, ldb,
-                                      beta, C, ldc, st);
-        return;
-    }
-    launch_tiles<T, WB, false>(ta, tb, false, 0, l2_map(false, fm, fn), m, n, k, alpha, A, lda, B, ldb, beta, C, ldc,
-                               st);
-    if (fm < ntm)   // partial last tile row (all tile columns)
-        launch_tiles<T, WB, true>(ta, tb, false, ntn, TileMap{2, ntm, fm, 0}, m, n, k, alpha, A, lda, B, ldb, beta,
-                                  C, ldc, st);
-    if (fn < ntn)   // partial last tile column (full tile rows only)
-        launch_tiles<T, WB, true>(ta, tb, false, fm, TileMap{3, ntm, 0, fn}, m, n, k, alpha, A, lda, B, ldb, beta,
-                                  C, ldc, st);
+    // optional timing of a lower launch; algorithmic work: the lower
+    // triangle, m (m + 1) k flop
+    const bool timed = prof && lower;
+    std::string name;
+    if (timed) name = std::string(prof) + "_t" + std::to_string(TILE);
+    ProfScope ps(timed ? name.c_str() : "", timed ? (double)m * (double)(m + 1) * (double)k : 0.0,
+                 timed ? st : nullptr);
+    if (!timed) ps.cancel();
+    const TileMap map = l2_map(lower, ntm, ntn);
+    if (vec)
+        launch_tiles<T, WB, true>(ta, tb, lower, 0, map, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, st);
+    else
+        launch_tiles<T, WB, false>(ta, tb, lower, 0, map, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, st);
 }
 
 template <typename T>
@@ -2356,19 +2357,8 @@ void build_grouped_gemm(const std::vector<GemmJob>& jobs, bool f32, bool ta, boo
         if (lower && j.m != j.n) throw std::invalid_argument("lower gemm needs a square output");
         const int64_t ntm = cdiv(j.m, TILE), ntn = cdiv(j.n, TILE);
         const bool vec = aligned_bytes(j.A, j.lda, elem) && aligned_bytes(j.B, j.ldb, elem);
-        if (!vec) {
-            add(ed, te, j, TileMap{lower ? 1 : 0, ntm, 0, 0}, lower ? ntm * (ntm + 1) / 2 : ntm * ntn);
-            continue;
-        }
-        const int64_t fm = j.m / TILE, fn = j.n / TILE;
-        if (lower) {
-            add(in, ti, j, TileMap{1, fm, 0, 0}, fm * (fm + 1) / 2);
-            if (fm < ntm) add(ed, te, j, TileMap{2, ntm, fm, 0}, ntm);
-        } else {
-            add(in, ti, j, TileMap{0, fm, 0, 0}, fm * fn);
-            if (fm < ntm) add(ed, te, j, TileMap{2, ntm, fm, 0}, ntn);
-            if (fn < ntn) add(ed, te, j, TileMap{3, ntm, 0, fn}, fm);
-        }
+        add(vec ? in : ed, vec ? ti : te, j, TileMap{lower ? 1 : 0, ntm, 0, 0},
+            lower ? ntm * (ntm + 1) / 2 : ntm * ntn);
     }
     const int base = (f32 ? 1 : 0) | (ta ? 2 : 0) | (tb ? 4 : 0) | (lower ? 8 : 0) | (wb == 4 ? 16 : 0);
     if (!in.empty()) {
@@ -2424,7 +2414,7 @@ void launch_grouped_gemm(const GemmLaunch& l, const GemmDesc* d_descs, int64_t g
 #define OMH_GG(F32, TA, TB, LO, W4, ED)                                                                    \
     case (F32) | ((TA) << 1) | ((TB) << 2) | ((LO) << 3) | ((W4) << 4) | ((ED) << 5):                    \
         k_gemm_grouped<typename std::conditional<(F32) != 0, float, double>::type, (TA) != 0, (TB) != 0,   \
-                       (LO) != 0, (W4) ? 4 : 2, (ED) != 0><<<grid, 256, 0, st>>>(d, l.ng, l.total);        \
+                       (LO) != 0, (W4) ? 4 : 2, (ED) == 0><<<grid, 256, 0, st>>>(d, l.ng, l.total);        \
         break;
 #define OMH_GG_OPS(F32, W4, ED) \
     OMH_GG(F32, 0, 0, 0, W4, ED) OMH_GG(F32, 1, 0, 0, W4, ED) OMH_GG(F32, 0, 1, 0, W4, ED) OMH_GG(F32, 0, 1, 1, W4, ED)
@@ -2540,35 +2530,25 @@ void gemm(bool ta, bool tb, bool lower, int64_t m, int64_t n, int64_t k, T alpha
     // per SIMD).  FP32: 128 x 128 tiles when they give at least ~2 waves of
     // workgroups over the 256 CUs.
     const int64_t big_tiles = lower ? cdiv(m, 128) * (cdiv(m, 128) + 1) / 2 : cdiv(m, 128) * cdiv(n, 128);
-    if (sizeof(T) == 4 && big_tiles >= 512)
-        gemm_launch<T, 4>(ta, tb, lower, vec, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, st, prof);
-    else
-        gemm_launch<T, 2>(ta, tb, lower, vec, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, st, prof);
+    if constexpr (sizeof(T) == 4)
+        if (big_tiles >= 512)
+            return gemm_launch<T, 4>(ta, tb, lower, vec, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, st, prof);
+    gemm_launch<T, 2>(ta, tb, lower, vec, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, st, prof);
 }
 
-// Split-K launch: interior tiles unguarded (16-byte aligned operands and
-// chunk starts), the partial last tile row and column guarded.
+// Split-K launch (vec: 16-byte aligned operands and chunk starts).
 template <typename T, bool TA, bool TB>
 static void splitk_tiles(bool vec, int64_t m, int64_t n, int64_t k, int64_t kc, int nsplit, const T* A, int64_t lda,
                          const T* B, int64_t ldb, T* W, hipStream_t st) {
     constexpr int WB = 2, TILE = 64;
     const int64_t ntm = cdiv(m, TILE), ntn = cdiv(n, TILE);
-    if (!vec) {
-        k_gemm_splitk<T, TA, TB, WB, true><<<dim3((unsigned)(ntm * ntn), nsplit), 256, 0, st>>>(
-            m, n, k, kc, A, lda, B, ldb, W, TileMap{0, ntm, 0, 0});
-        OMH_LAUNCH_CHECK();
-        return;
-    }
-    const int64_t fm = m / TILE, fn = n / TILE;
-    if (fm * fn > 0)
-        k_gemm_splitk<T, TA, TB, WB, false><<<dim3((unsigned)(fm * fn), nsplit), 256, 0, st>>>(
-            m, n, k, kc, A, lda, B, ldb, W, TileMap{0, fm, 0, 0});
-    if (fm < ntm)   // partial last tile row (all tile columns)
-        k_gemm_splitk<T, TA, TB, WB, true><<<dim3((unsigned)ntn, nsplit), 256, 0, st>>>(
-            m, n, k, kc, A, lda, B, ldb, W, TileMap{2, ntm, fm, 0});
-    if (fn < ntn && fm > 0)   // partial last tile column (full tile rows only)
-        k_gemm_splitk<T, TA, TB, WB, true><<<dim3((unsigned)fm, nsplit), 256, 0, st>>>(
-            m, n, k, kc, A, lda, B, ldb, W, TileMap{3, ntm, 0, fn});
+    const dim3 grid((unsigned)(ntm * ntn), nsplit);
+    if (vec)
+        k_gemm_splitk<T, TA, TB, WB, true><<<grid, 256, 0, st>>>(m, n, k, kc, A, lda, B, ldb, W,
+                                                                 TileMap{0, ntm, 0, 0});
+    else
+        k_gemm_splitk<T, TA, TB, WB, false><<<grid, 256, 0, st>>>(m, n, k, kc, A, lda, B, ldb, W,
+                                                                  TileMap{0, ntm, 0, 0});
     OMH_LAUNCH_CHECK();
 }
 
