@@ -3330,6 +3330,214 @@ __global__ void __launch_bounds__(256) k_solve_group(const T* __restrict__ L, in
     }
 }
 
+// k_solve_group for two right-hand sides a workgroup, where the time is that
+// of bringing the group's ten 256 x 256 blocks to the CU (64 B a clock: 17 us
+// FP32): 16 waves, each block read once in whole 16-byte loads that lie side
+// by side, the next block's in flight over the reduction of the current one.
+// Forward (A X): a lane takes 4 rows, a wave 16 of the 256 columns; the
+// waves' partial sums are added in LDS.  Backward (A^T X): a wave takes 16
+// columns of A, 16 lanes along each; their sums meet in DPP rotations.
+// Groups of whole blocks, 16-byte aligned columns (k_solve_group the others).
+// 17926 unknowns, 128 right-hand sides: 48 us forward and 41 us backward a
+// group (one thread a row over all of k: 68 and 77 us), FP64 82 and 69 us
+// (109 and 132 us).
+constexpr int SG_THREADS = 1024, SG_WAVES = SG_THREADS / 64;
+
+template <int N>
+__device__ __forceinline__ float row_ror(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x120 + N, 0xf, 0xf, true));
+}
+template <int N>
+__device__ __forceinline__ double row_ror(double v) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)b, 0x120 + N, 0xf, 0xf, true);
+    const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), 0x120 + N, 0xf, 0xf, true);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+template <typename T, bool BACK>
+__global__ void __launch_bounds__(SG_THREADS) k_solve_pair(const T* __restrict__ L, int64_t lda,
+                                                           const T* __restrict__ Dinv, int64_t k0, int64_t gend,
+                                                           T* __restrict__ W, int64_t ldw, int64_t r, WSplit ws) {
+    constexpr int SV = 2, NB = FACT_NB, G = SOLVE_GROUP * FACT_NB;
+    constexpr int VW = 16 / sizeof(T), NV = 4 / VW;   // elements and loads of 4 values
+    constexpr int PASS = sizeof(T) / 4;               // passes over a block (the registers hold half of FP64)
+    constexpr int U = 16 / PASS;                      // 4-value loads of a pass
+    typedef T vec_t __attribute__((ext_vector_type(VW)));
+    __shared__ __align__(16) T Wg[G][SV];
+    __shared__ __align__(16) T red[BACK ? 1 : SG_WAVES][NB][SV];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t c0 = (int64_t)blockIdx.x * SV;
+    const int nc = (int)min<int64_t>(SV, r - c0);
+    const int g = (int)(gend - k0);
+    for (int e = tid; e < g * SV; e += SG_THREADS) {
+        const int i = e % g, c = e / g;
+        Wg[i][c] = c < nc ? W[k0 + i + (c0 + c) * ldw] : T(0);
+    }
+    const int nbk = g / NB;
+    // value q of load u of pass h in block (b2, b): forward rows 4 lane + q,
+    // column 16 wave + (U h + u); backward column 16 wave + 4 t + lane / 16
+    // of A, rows 64 s + 4 (lane % 16) + q, with (t, s) of U h + u
+    T a[U][4];
+    auto load = [&](int b, int b2, int h) {
+        const bool diag = b == b2;
+        const T* A = diag ? Dinv + ((size_t)(k0 / NB) + b) * NB * NB
+                          : (BACK ? L + (k0 + b * NB) + (k0 + b2 * NB) * lda : L + (k0 + b2 * NB) + (k0 + b * NB) * lda);
+        const int64_t ld = diag ? NB : lda;
+        const unsigned lo = BACK ? 4 * (lane & 15) + (unsigned)(lane >> 4) * (unsigned)ld : 4 * lane;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int x = U * h + u;
+            const T* Au = BACK ? A + 64 * (x & 3) + (int64_t)(16 * wave + 4 * (x >> 2)) * ld
+                               : A + (int64_t)(16 * wave + x) * ld;
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                const vec_t w = *reinterpret_cast<const vec_t*>(Au + lo + v * VW);
+#pragma unroll
+                for (int q = 0; q < VW; ++q) a[u][v * VW + q] = w[q];
+            }
+        }
+    };
+    int b = BACK ? nbk - 1 : 0, b2 = b;
+    load(b, b2, 0);
+    __syncthreads();
+    for (;;) {
+        // the block after this one
+        int nb = b, nb2;
+        bool more = true;
+        if (BACK) {
+            nb2 = b2 == b ? 0 : b2 + 1;
+            if (nb2 >= b) {
+                nb = b - 1;
+                nb2 = nb;
+                more = nb >= 0;
+            }
+        } else {
+            nb2 = b2 + 1;
+            if (nb2 >= nbk) {
+                nb = b + 1;
+                nb2 = nb;
+                more = nb < nbk;
+            }
+        }
+        constexpr int NA = 4;   // forward: rows of a lane; backward: columns
+        T acc[NA][SV];
+#pragma unroll
+        for (int q = 0; q < NA; ++q)
+#pragma unroll
+            for (int c = 0; c < SV; ++c) acc[q][c] = T(0);
+        const T (*X)[SV] = &Wg[b * NB];
+#pragma unroll
+        for (int h = 0; h < PASS; ++h) {
+            if (!BACK) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const T x0 = X[16 * wave + U * h + u][0], x1 = X[16 * wave + U * h + u][1];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        acc[q][0] = fma(a[u][q], x0, acc[q][0]);
+                        acc[q][1] = fma(a[u][q], x1, acc[q][1]);
+                    }
+                    if (u % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // X a few rows at a time
+                }
+            } else {
+#pragma unroll
+                for (int sx = 0; sx < 4; ++sx) {
+                    T x[4][SV];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+#pragma unroll
+                        for (int c = 0; c < SV; ++c) x[q][c] = X[64 * sx + 4 * (lane & 15) + q][c];
+#pragma unroll
+                    for (int t = 0; t < U / 4; ++t)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q)
+#pragma unroll
+                            for (int c = 0; c < SV; ++c) {
+                                const int o = t + h * (U / 4);
+                                acc[o][c] = fma(a[4 * t + sx][q], x[q][c], acc[o][c]);
+                            }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            // into the registers just used (kept behind them)
+            __builtin_amdgcn_sched_barrier(0);
+            if (h + 1 < PASS) load(b, b2, h + 1);
+            else load(more ? nb : b, more ? nb2 : b2, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (!BACK) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int c = 0; c < SV; ++c) red[wave][4 * lane + q][c] = acc[q][c];
+            __syncthreads();   // the partial sums are there, X has been read
+            if (tid < NB * SV) {
+                const int i = tid / SV, c = tid % SV;
+                T v = T(0);
+#pragma unroll
+                for (int w = 0; w < SG_WAVES; ++w) v += red[w][i][c];
+                if (b2 == b) Wg[b * NB + i][c] = v;
+                else Wg[b2 * NB + i][c] -= v;
+            }
+            __syncthreads();
+        } else {
+            T v = T(0);
+            const int j = lane & 15;   // lanes 0..7 of a group take one sum each
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int c = 0; c < SV; ++c) {
+                    T x = acc[t][c];
+                    x += row_ror<8>(x);
+                    x += row_ror<4>(x);
+                    x += row_ror<2>(x);
+                    x += row_ror<1>(x);
+                    if (j == t * SV + c) v = x;
+                }
+            if (b2 == b) __syncthreads();   // X has been read
+            const int i = 16 * wave + 4 * (j / SV) + (lane >> 4);
+            if (j < 4 * SV) {
+                T& w = Wg[b2 * NB + i][j % SV];
+                w = b2 == b ? v : w - v;
+            }
+            if (b2 == b || nb != b) __syncthreads();   // the next block's X is complete
+        }
+        if (!more) break;
+        b = nb;
+        b2 = nb2;
+    }
+    for (int e = tid; e < g * SV; e += SG_THREADS) {
+        const int i = e % g, c = e / g;
+        if (c < nc) W[k0 + i + (c0 + c) * ldw] = Wg[i][c];
+    }
+    if (sizeof(T) == 4 && ws.h) {   // FP32 solves only: the split copy for the products that follow
+        __shared__ float mx[SV][SG_WAVES];
+#pragma unroll
+        for (int c = 0; c < SV; ++c) {
+            float m = 0.f;
+            for (int i = tid; i < g; i += SG_THREADS) m = fmaxf(m, fabsf((float)Wg[i][c]));
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+            if (lane == 0) mx[c][wave] = m;
+        }
+        __syncthreads();
+        for (int e = tid; e < g * SV; e += SG_THREADS) {
+            const int i = e % g, c = e / g;
+            float m = 0.f;
+            for (int w = 0; w < SG_WAVES; ++w) m = fmaxf(m, mx[c][w]);
+            int ex = 0;
+            if (m > 0.f) (void)frexpf(m, &ex);   // max = f 2^ex, f in [0.5, 1)
+            const float x = (float)Wg[i][c] * ldexpf(1.f, -ex);
+            const _Float16 hx = (_Float16)x;
+            const int64_t o = ((int64_t)(i / 32) * ws.rp + c0 + c) * 32 + i % 32;
+            ws.h[o] = hx;
+            ws.l[o] = (_Float16)(x - (float)hx);
+            if (i == 0) ws.tw[c0 + c] = ldexpf(1.f, ex);
+        }
+    }
+}
+
 // Row intervals [start, start + len) of a split solve product, cut into
 // tiles of `tile` rows: tile x lies in the interval k with tile0[k] <= x <
 // tile0[k + 1].
@@ -3683,15 +3891,49 @@ static void sym_solve_impl(const T* L, int64_t n, int64_t lda, const void* work,
         return cdiv(rows, 64) * cdiv(r, 64) >= 1024;
     };
     // strips of 2 right-hand sides up to 1024 of them (128 workgroups for
-    // 256; 8-wide strips took twice as long per group at 256), else 8
+    // 256; 8-wide strips took twice as long per group at 256); beyond, GEMMs
+    // (FP64) or strips of 8
     const bool narrow = r <= 1024;
+    T* tmp = nullptr;   // a block of rows of W (not under capture: the scratch may have to grow)
+    if (!narrow && sizeof(T) == 8) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        OMH_HIP(hipStreamIsCapturing(st, &cap));
+        if (cap == hipStreamCaptureStatusNone)
+            tmp = (T*)scratch(SCR_SOLVE_TMP, sizeof(T) * (size_t)FACT_NB * (size_t)r, st);
+    }
     auto group_solve = [&](bool back, int64_t k0, int64_t gend, bool split) {
         WSplit ws;
         if (split) ws = sb->ws;
-        if (narrow) {
+        const bool whole = (gend - k0) % FACT_NB == 0 && aligned_for_vec(L, lda) && aligned_for_vec(Dinv, 4) &&
+                           lda < (int64_t(1) << 28);
+        if (narrow && whole) {
+            const unsigned g = (unsigned)cdiv(r, 2);
+            if (back) k_solve_pair<T, true><<<g, SG_THREADS, 0, st>>>(L, lda, Dinv, k0, gend, W, ldw, r, ws);
+            else k_solve_pair<T, false><<<g, SG_THREADS, 0, st>>>(L, lda, Dinv, k0, gend, W, ldw, r, ws);
+        } else if (narrow) {
             const unsigned g = (unsigned)cdiv(r, 2);
             if (back) k_solve_group<T, true, 2><<<g, 256, 0, st>>>(L, lda, Dinv, k0, gend, W, ldw, r, ws);
             else k_solve_group<T, false, 2><<<g, 256, 0, st>>>(L, lda, Dinv, k0, gend, W, ldw, r, ws);
+        } else if (tmp) {
+            // more right-hand sides than strips can use: the same block
+            // products as whole GEMMs (8136 unknowns, as many right-hand
+            // sides: about 0.3 ms a group against 1.17 ms forward and 0.52 ms
+            // backward for strips of 8, which read L for each strip)
+            const int nbk = (int)cdiv(gend - k0, FACT_NB);
+            for (int bi = 0; bi < nbk; ++bi) {
+                const int64_t kb = k0 + (int64_t)(back ? nbk - 1 - bi : bi) * FACT_NB;
+                const int64_t nb = std::min<int64_t>(FACT_NB, gend - kb);
+                gemm<T>(back, false, false, nb, r, nb, T(1), Dinv + (size_t)(kb / FACT_NB) * FACT_NB * FACT_NB, FACT_NB,
+                        W + kb, ldw, T(0), tmp, FACT_NB, st);
+                k_copy<T><<<grid_for(nb * r), 256, 0, st>>>(tmp, FACT_NB, W + kb, ldw, nb, r);
+                OMH_LAUNCH_CHECK();
+                if (back && kb > k0)
+                    gemm<T>(true, false, false, kb - k0, r, nb, T(-1), L + kb + k0 * lda, lda, W + kb, ldw, T(1),
+                            W + k0, ldw, st);
+                if (!back && kb + nb < gend)
+                    gemm<T>(false, false, false, gend - kb - nb, r, nb, T(-1), L + kb + nb + kb * lda, lda, W + kb,
+                            ldw, T(1), W + kb + nb, ldw, st);
+            }
         } else {
             const unsigned g = (unsigned)cdiv(r, 8);
             if (back) k_solve_group<T, true, 8><<<g, 256, 0, st>>>(L, lda, Dinv, k0, gend, W, ldw, r, ws);

@@ -1,0 +1,86 @@
+"""Triangular solves of the stored factor over the paths a group of four
+256-blocks can take: whole groups (k_solve_pair), partial groups and odd
+leading dimensions (k_solve_group), more than 1024 right-hand sides (block
+GEMMs for FP64); FP32 split products and their scale cache."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def om():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import openmeeg_amd
+    return openmeeg_amd
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n,r,pad", [(256, 1, 0), (255, 3, 1), (1024, 2, 0), (1024, 5, 3), (1025, 7, 3), (1536, 64, 0),
+                                     (2048, 33, 4), (2300, 130, 4), (1280, 1030, 0), (1300, 1100, 1)])
+def test_solve_residual(om, n, r, pad, dtype):
+    import torch
+    from openmeeg_amd import _lib
+    lib = _lib.lib()
+    rng = np.random.default_rng(n + r)
+    t = torch.float64 if dtype == np.float64 else torch.float32
+    size = np.dtype(dtype).itemsize
+    # quasi-definite: +/- diagonal blocks, well conditioned
+    A = rng.standard_normal((n, n)) / np.sqrt(n)
+    A = 0.25 * (A + A.T) + np.diag(np.where(np.arange(n) < n // 2, 2.0, -2.0))
+    ld, ldb = n + pad, n + pad
+    dA = torch.zeros((n, ld), dtype=t, device="cuda")
+    dA[:, :n] = torch.from_numpy(A.astype(dtype))
+    Ad = dA[:, :n].double().clone()
+    B = rng.standard_normal((r, ldb))
+    dB = torch.from_numpy(B.astype(dtype)).cuda()
+    B0 = dB.double().clone()
+    work = torch.zeros(int(lib.omh_factor_workspace_bytes(n, size)), dtype=torch.uint8, device="cuda")
+    info = C.c_int32()
+    f = lib.omh_sym_factor_f64 if size == 8 else lib.omh_sym_factor_f32
+    s = lib.omh_sym_solve_f64 if size == 8 else lib.omh_sym_solve_f32
+    p = lambda x: C.c_void_p(x.data_ptr())
+    _lib.check(f(p(dA), n, ld, p(work), C.byref(info), C.c_void_p(0)))
+    assert info.value == 0
+    _lib.check(s(p(dA), n, ld, p(work), p(dB), ldb, r, C.c_void_p(0)))
+    torch.cuda.synchronize()
+    X = dB[:, :n].double()
+    res = (X @ Ad - B0[:, :n]).norm(dim=1) / (Ad.abs().sum(1).max() * X.norm(dim=1))
+    # ||b - A x|| <= c n eps ||A|| ||x|| (backward stability of the factor and
+    # both substitutions, explicit 256-block inverses of condition < 10)
+    assert float(res.max()) < 10 * np.sqrt(n) * np.finfo(dtype).eps
+    if pad:
+        assert torch.equal(dB[:, n:].double(), B0[:, n:])
+
+
+def test_split_products_scale_cache_many_rhs(om, monkeypatch):
+    """Enough right-hand sides that the split products run (1024 tiles of
+    64 x 64 and more): cached scales against scales formed by every solve,
+    bitwise, on a factor whose order is not a multiple of 4."""
+    import torch
+    from openmeeg_amd.api import _head_mat_device, factor
+    from openmeeg_amd import spheres as S
+    g = om.make_nested_geometry(S.nested_sphere_meshes(12, (0.87, 0.92, 1.0)), (1.0, 0.0125, 1.0))
+    n, r = g.size, 700
+    assert n % 4 == 2
+    H = _head_mat_device(g, far_field=True)
+    F = factor(H, n, "mixed16", structure=g.factor_segments(), n_positive=n - g.n_vertex_unknowns,
+               order=g.factor_order())
+    assert F.ld % 4 == 0
+    B = torch.from_numpy(np.random.default_rng(4).standard_normal(n * r)).cuda()
+    X = {}
+    for mode in ("cache", "none"):
+        if mode == "none":
+            monkeypatch.setenv("OMH_SOLVE_SCALE_CACHE", "0")
+        X[mode] = B.clone()
+        F.solve(X[mode], r, max_iter=10, tol=1e-12)
+        torch.cuda.synchronize()
+        monkeypatch.delenv("OMH_SOLVE_SCALE_CACHE", raising=False)
+    assert F.iterations >= 2
+    assert torch.equal(X["cache"], X["none"])
+    res = torch.linalg.norm(B.view(r, n) - X["cache"].view(r, n) @ H.view(n, n)) / torch.linalg.norm(B)
+    assert float(res) < 1e-12
