@@ -64,33 +64,19 @@ struct Frame {
     int level;
 };
 
-// Integrator::integrate (integrator.h:44-48) with the adaptive recursion of
-// integrator.h:69-93 unrolled onto an explicit stack; the child results are
-// summed in the reference's order.
+// The adaptive recursion of integrator.h:69-93 below a triangle whose four
+// children's integrals are known and do not satisfy the tolerance, unrolled
+// onto an explicit stack; the child results are summed in the reference's
+// order.
 template <int NC, class F>
-__device__ void integrate(const F& f, int order, int levels, double tol, const d3 P[3], double area, double* res) {
-    double coarse[NC];
-    tri_integration<NC>(f, order, P[0], P[1], P[2], area, coarse);
-    if (levels <= 0) {
-        for (int c = 0; c < NC; ++c) res[c] = coarse[c];
-        return;
-    }
+__device__ void integrate_deep(const F& f, int order, int levels, double tol, const d3 P[3], double area,
+                               const double (*integ0)[NC], double* res) {
     Frame<NC> st[ADAPT_MAX_FRAMES];
     int top = 0;
     st[0].P[0] = P[0]; st[0].P[1] = P[1]; st[0].P[2] = P[2];
     st[0].area = area;
-    double refined[NC];
-    for (int c = 0; c < NC; ++c) refined[c] = 0.0;
-    for (int i = 0; i < 4; ++i) {
-        d3 C[3];
-        child_tri(P, i, C);
-        tri_integration<NC>(f, order, C[0], C[1], C[2], 0.25 * area, st[0].integ[i]);
-        for (int c = 0; c < NC; ++c) refined[c] += st[0].integ[i][c];
-    }
-    if (converged<NC>(coarse, refined, tol)) {
-        for (int c = 0; c < NC; ++c) res[c] = refined[c];
-        return;
-    }
+    for (int i = 0; i < 4; ++i)
+        for (int c = 0; c < NC; ++c) st[0].integ[i][c] = integ0[i][c];
     st[0].level = levels;
     st[0].child = 0;
     for (int c = 0; c < NC; ++c) st[0].sum[c] = 0.0;
@@ -134,6 +120,30 @@ __device__ void integrate(const F& f, int order, int levels, double tol, const d
             ++top;
         }
     }
+}
+
+// Integrator::integrate (integrator.h:44-48).
+template <int NC, class F>
+__device__ void integrate(const F& f, int order, int levels, double tol, const d3 P[3], double area, double* res) {
+    double coarse[NC];
+    tri_integration<NC>(f, order, P[0], P[1], P[2], area, coarse);
+    if (levels <= 0) {
+        for (int c = 0; c < NC; ++c) res[c] = coarse[c];
+        return;
+    }
+    double integ[4][NC], refined[NC];
+    for (int c = 0; c < NC; ++c) refined[c] = 0.0;
+    for (int i = 0; i < 4; ++i) {
+        d3 C[3];
+        child_tri(P, i, C);
+        tri_integration<NC>(f, order, C[0], C[1], C[2], 0.25 * area, integ[i]);
+        for (int c = 0; c < NC; ++c) refined[c] += integ[i][c];
+    }
+    if (converged<NC>(coarse, refined, tol)) {
+        for (int c = 0; c < NC; ++c) res[c] = refined[c];
+        return;
+    }
+    integrate_deep<NC>(f, order, levels, tol, P, area, integ, res);
 }
 
 }  // namespace omh

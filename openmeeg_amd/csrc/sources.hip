@@ -70,6 +70,55 @@ struct DerivativeFn {           // PotentialDerivative (analytics.h:140-150)
     }
 };
 
+// Both integrands over a triangle and its four children (child_tri's order)
+// with the 16-point rule: what every pair needs before the adaptive
+// recursion's first test, and all that a pair away from the dipole needs.
+// On the triangle's plane x.n (x = r - r0) is the constant h and x, q.x and
+// the barycentric coordinates are linear in the rule's, so a point takes one
+// reciprocal root and about 30 FP64 instructions for both integrands (120
+// through the functors, point by point).  D[0], V[0]: the triangle; D[1 + c],
+// V[1 + c]: child c.
+__device__ __forceinline__ void fan_integrals(d3 a0, d3 e1, d3 e2, d3 q, d3 n, double area, double (*D)[3],
+                                              double* V) {
+    const double m3h = -3.0 * dot(a0, n), qn = dot(q, n);
+    const double qa = dot(q, a0), q1 = dot(q, e1), q2 = dot(q, e2);
+#pragma unroll
+    for (int t = 0; t < 5; ++t) {
+        // vertices A, A + u, A + v of the sub-triangle in units of e1 and e2:
+        // the triangle, then (P0, m1, m2), (m0, P1, m2), (m0, m1, P2),
+        // (m0, m1, m2) with m0 = (P1 + P2) / 2, m1 = (P2 + P0) / 2, m2 = (P0 + P1) / 2
+        const double A1 = t >= 2 ? 0.5 : 0.0, A2 = t >= 2 ? 0.5 : 0.0;
+        const double u1 = t == 0 ? 1.0 : t == 1 ? 0.0 : t == 2 ? 0.5 : -0.5;
+        const double u2 = t == 0 ? 0.0 : t == 1 ? 0.5 : t == 2 ? -0.5 : 0.0;
+        const double v1 = t == 0 ? 0.0 : t == 1 ? 0.5 : t == 3 ? -0.5 : 0.0;
+        const double v2 = t == 0 ? 1.0 : t == 1 ? 0.0 : t == 3 ? 0.5 : -0.5;
+        const d3 A = add(a0, add(scl(A1, e1), scl(A2, e2)));
+        const d3 u = add(scl(u1, e1), scl(u2, e2)), v = add(scl(v1, e1), scl(v2, e2));
+        const double qA = qa + A1 * q1 + A2 * q2, qu = u1 * q1 + u2 * q2, qv = v1 * q1 + v2 * q2;
+        double s0 = 0.0, s1 = 0.0, s2 = 0.0, sp = 0.0;
+#pragma unroll 4
+        for (int i = 0; i < 16; ++i) {
+            const double b1 = c_rules[3][i][1], b2 = c_rules[3][i][2], w = c_rules[3][i][3];
+            const d3 x = mk(fma(b2, v.x, fma(b1, u.x, A.x)), fma(b2, v.y, fma(b1, u.y, A.y)),
+                            fma(b2, v.z, fma(b1, u.z, A.z)));
+            const double qx = fma(b2, qv, fma(b1, qu, qA));
+            const double ir = rsqrt_pos(dot(x, x)), ir2 = ir * ir, wi3 = w * (ir * ir2);
+            const double g = fma(m3h, qx * ir2, qn) * wi3;
+            s0 += g;
+            s1 = fma(g, b1, s1);
+            s2 = fma(g, b2, s2);
+            sp = fma(qx, wi3, sp);
+        }
+        // from the sub-triangle's barycentric coordinates to the triangle's
+        const double ar = t == 0 ? area : 0.25 * area;
+        const double l1 = A1 * s0 + u1 * s1 + v1 * s2, l2 = A2 * s0 + u2 * s1 + v2 * s2;
+        D[t][0] = ar * (s0 - l1 - l2);
+        D[t][1] = ar * l1;
+        D[t][2] = ar * l2;
+        V[t] = ar * sp;
+    }
+}
+
 // One (triangle, dipole) pair of one mesh: the P1 derivative integral into
 // W[(k*nd + s)*nt + t] and, for non-barrier meshes, the P0 potential
 // integral added to out(row(t), s).
@@ -91,13 +140,32 @@ __global__ void __launch_bounds__(256) k_dsm_pairs(const TriRec* __restrict__ tr
         const TriRec& T = tri[t0 + t];
         const d3 P[3] = {ld3(T.p[0]), ld3(T.p[1]), ld3(T.p[2])};
         const d3 pos = ld3(dip + 6 * sg), mom = ld3(dip + 6 * sg + 3);
-        DerivativeFn fd;
-        fd.init(T, pos, mom);
-        integrate<3>(fd, order, levels, tol, P, T.area, v3v);
+        double pv = 0.0;
+        if (order == 3 && levels > 0) {
+            double D[5][3], V[5], dr[3], vr[1];
+            fan_integrals(sub(P[0], pos), sub(P[1], P[0]), sub(P[2], P[0]), mom, ld3(T.n), T.area, D, V);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) dr[c] = D[1][c] + D[2][c] + D[3][c] + D[4][c];
+            vr[0] = V[1] + V[2] + V[3] + V[4];
+            const bool cd = converged<3>(D[0], dr, tol), cv = !with_pot || converged<1>(V, vr, tol);
+            for (int c = 0; c < 3; ++c) v3v[c] = dr[c];
+            pv = vr[0];
+            if (!cd) {
+                DerivativeFn fd;
+                fd.init(T, pos, mom);
+                integrate_deep<3>(fd, order, levels, tol, P, T.area, D + 1, v3v);
+            }
+            if (!cv) {
+                const double vc[4][1] = {{V[1]}, {V[2]}, {V[3]}, {V[4]}};
+                integrate_deep<1>(PotentialFn{pos, mom}, order, levels, tol, P, T.area, vc, &pv);
+            }
+        } else {
+            DerivativeFn fd;
+            fd.init(T, pos, mom);
+            integrate<3>(fd, order, levels, tol, P, T.area, v3v);
+            if (with_pot) integrate<1>(PotentialFn{pos, mom}, order, levels, tol, P, T.area, &pv);
+        }
         if (with_pot) {
-            PotentialFn fp{pos, mom};
-            double pv;
-            integrate<1>(fp, order, levels, tol, P, T.area, &pv);
             const int64_t r = dev_index(L, tri_unk0 + t);
             out[r + sg * ld_out] += pv * cP[sg * nm + mesh];
         }
