@@ -127,7 +127,11 @@ class EEGForward:
         D = _dev_f64(n * max(nd, 1))
         check(lib().omh_dip_source_mat(g._h, _ptr(dip), nd, doms, self.order, 0, 0.0, _ptr(D), n,
                                        ORDER_TRIANGLES_FIRST, _stream()))
-        F = factor(H, n, self.precision)
+        # the pipelines' block structure and mesh-by-mesh order: the factor and
+        # the solves skip the blocks that are zero
+        structure = g.factor_segments()
+        F = factor(H, n, self.precision, structure=structure,
+                   order=g.factor_order() if structure is not None else None)
         Y = self._E.clone()
         F.solve(Y, ne, max_iter=self.max_refine, tol=self.refine_tol)
         G = _dev_f64(ne * max(nd, 1))
