@@ -75,13 +75,16 @@ struct DerivativeFn {           // PotentialDerivative (analytics.h:140-150)
 // recursion's first test, and all that a pair away from the dipole needs.
 // On the triangle's plane x.n (x = r - r0) is the constant h and x, q.x and
 // the barycentric coordinates are linear in the rule's, so a point takes one
-// reciprocal root and about 30 FP64 instructions for both integrands (120
+// reciprocal root and about 35 FP64 instructions for both integrands (120
 // through the functors, point by point).  D[0], V[0]: the triangle; D[1 + c],
 // V[1 + c]: child c.
-__device__ __forceinline__ void fan_integrals(d3 a0, d3 e1, d3 e2, d3 q, d3 n, double area, double (*D)[3],
+// The rule's coordinates are given to 15 digits and add up to 1 + d with d up
+// to 2e-15: the point is sum b P, so x, q.x and x.n carry d times the vertex.
+__device__ __forceinline__ void fan_integrals(d3 P0, d3 r0, d3 e1, d3 e2, d3 q, d3 n, double area, double (*D)[3],
                                               double* V) {
-    const double m3h = -3.0 * dot(a0, n), qn = dot(q, n);
-    const double qa = dot(q, a0), q1 = dot(q, e1), q2 = dot(q, e2);
+    const d3 a0 = sub(P0, r0);
+    const double m3h = -3.0 * dot(a0, n), qn = dot(q, n), m3n = -3.0 * dot(P0, n);
+    const double qa = dot(q, a0), q1 = dot(q, e1), q2 = dot(q, e2), qP = dot(q, P0);
 #pragma unroll
     for (int t = 0; t < 5; ++t) {
         // vertices A, A + u, A + v of the sub-triangle in units of e1 and e2:
@@ -92,29 +95,29 @@ __device__ __forceinline__ void fan_integrals(d3 a0, d3 e1, d3 e2, d3 q, d3 n, d
         const double u2 = t == 0 ? 0.0 : t == 1 ? 0.5 : t == 2 ? -0.5 : 0.0;
         const double v1 = t == 0 ? 0.0 : t == 1 ? 0.5 : t == 3 ? -0.5 : 0.0;
         const double v2 = t == 0 ? 1.0 : t == 1 ? 0.0 : t == 3 ? 0.5 : -0.5;
-        const d3 A = add(a0, add(scl(A1, e1), scl(A2, e2)));
+        const d3 off = add(scl(A1, e1), scl(A2, e2)), A = add(a0, off), Q = add(P0, off);
         const d3 u = add(scl(u1, e1), scl(u2, e2)), v = add(scl(v1, e1), scl(v2, e2));
-        const double qA = qa + A1 * q1 + A2 * q2, qu = u1 * q1 + u2 * q2, qv = v1 * q1 + v2 * q2;
+        const double qo = A1 * q1 + A2 * q2, qA = qa + qo, qQ = qP + qo, qu = u1 * q1 + u2 * q2, qv = v1 * q1 + v2 * q2;
         double s0 = 0.0, s1 = 0.0, s2 = 0.0, sp = 0.0;
 #pragma unroll 4
         for (int i = 0; i < 16; ++i) {
-            const double b1 = c_rules[3][i][1], b2 = c_rules[3][i][2], w = c_rules[3][i][3];
-            const d3 x = mk(fma(b2, v.x, fma(b1, u.x, A.x)), fma(b2, v.y, fma(b1, u.y, A.y)),
-                            fma(b2, v.z, fma(b1, u.z, A.z)));
-            const double qx = fma(b2, qv, fma(b1, qu, qA));
+            const double b0 = c_rules[3][i][0], b1 = c_rules[3][i][1], b2 = c_rules[3][i][2], w = c_rules[3][i][3];
+            const double d = (b1 + b2) + b0 - 1.0;
+            const d3 x = mk(fma(b2, v.x, fma(b1, u.x, fma(d, Q.x, A.x))), fma(b2, v.y, fma(b1, u.y, fma(d, Q.y, A.y))),
+                            fma(b2, v.z, fma(b1, u.z, fma(d, Q.z, A.z))));
+            const double qx = fma(b2, qv, fma(b1, qu, fma(d, qQ, qA)));
             const double ir = rsqrt_pos(dot(x, x)), ir2 = ir * ir, wi3 = w * (ir * ir2);
-            const double g = fma(m3h, qx * ir2, qn) * wi3;
-            s0 += g;
+            const double g = fma(fma(d, m3n, m3h), qx * ir2, qn) * wi3;
+            s0 = fma(g, b0, s0);
             s1 = fma(g, b1, s1);
             s2 = fma(g, b2, s2);
             sp = fma(qx, wi3, sp);
         }
         // from the sub-triangle's barycentric coordinates to the triangle's
         const double ar = t == 0 ? area : 0.25 * area;
-        const double l1 = A1 * s0 + u1 * s1 + v1 * s2, l2 = A2 * s0 + u2 * s1 + v2 * s2;
-        D[t][0] = ar * (s0 - l1 - l2);
-        D[t][1] = ar * l1;
-        D[t][2] = ar * l2;
+        D[t][0] = ar * ((1 - A1 - A2) * s0 + (1 - A1 - u1 - A2 - u2) * s1 + (1 - A1 - v1 - A2 - v2) * s2);
+        D[t][1] = ar * (A1 * s0 + (A1 + u1) * s1 + (A1 + v1) * s2);
+        D[t][2] = ar * (A2 * s0 + (A2 + u2) * s1 + (A2 + v2) * s2);
         V[t] = ar * sp;
     }
 }
@@ -143,7 +146,7 @@ __global__ void __launch_bounds__(256) k_dsm_pairs(const TriRec* __restrict__ tr
         double pv = 0.0;
         if (order == 3 && levels > 0) {
             double D[5][3], V[5], dr[3], vr[1];
-            fan_integrals(sub(P[0], pos), sub(P[1], P[0]), sub(P[2], P[0]), mom, ld3(T.n), T.area, D, V);
+            fan_integrals(P[0], pos, sub(P[1], P[0]), sub(P[2], P[0]), mom, ld3(T.n), T.area, D, V);
 #pragma unroll
             for (int c = 0; c < 3; ++c) dr[c] = D[1][c] + D[2][c] + D[3][c] + D[4][c];
             vr[0] = V[1] + V[2] + V[3] + V[4];
