@@ -574,11 +574,12 @@ class Factor:
 
     A mixed-precision factor whose refinement does not converge (the FP32
     factor too coarse for the matrix) is replaced by the FP64 factor of the
-    FP64 matrix when fallback_fp64 is set (then `fell_back` is True);
-    otherwise solve() raises NotConverged."""
+    FP64 matrix when fallback_fp64 is set (then `fell_back` is True; `keep`:
+    of a copy, the FP64 matrix stays as it is); otherwise solve() raises
+    NotConverged."""
 
     def __init__(self, L, n, work, precision, H64=None, structure=None, fallback_fp64=True, ipiv=None,
-                 n_positive=None, order=None, ld=None):
+                 n_positive=None, order=None, ld=None, keep=False):
         self.L, self.n, self.work, self.precision, self.H64 = L, n, work, precision, H64
         self.ld = n if ld is None else ld   # leading dimension of L
         self.ipiv = ipiv
@@ -587,6 +588,7 @@ class Factor:
         self.fell_back = False
         self.pivoted = precision == "lu"
         self.fallback_fp64 = fallback_fp64
+        self.keep = keep
         self.n_positive = n_positive
         self._raw_structure = structure
         self._structure = _block_args(structure)
@@ -597,12 +599,12 @@ class Factor:
 
     def _refactor_fp64(self):
         """Factor the FP64 matrix in place (it is no longer needed for
-        residuals) and drop the FP32 factor; the LU with partial pivoting
-        when the pivot-free factorisation breaks down on it."""
+        residuals; with `keep` a copy) and drop the FP32 factor; the LU with
+        partial pivoting when the pivot-free factorisation breaks down on it."""
         H = self.H64
-        backup = H.clone() if self.n_positive is not None else None
+        backup = H.clone() if self.n_positive is not None and not self.keep else None
         F = factor(H, self.n, "fp64", structure=self._raw_structure, n_positive=self.n_positive,
-                   rebuild=(lambda: backup) if backup is not None else None)
+                   rebuild=(lambda: backup) if backup is not None else None, keep=self.keep)
         self.L, self.work, self.precision, self.H64, self.ipiv = F.L, F.work, F.precision, None, F.ipiv
         self.order, self._fstructure, self.ld = F.order, F._fstructure, F.ld
         self.pivoted = F.pivoted
@@ -723,7 +725,8 @@ def _lu_factor(Hdev, n):
     return Factor(Hdev, n, work, "lu", ipiv=ipiv)
 
 
-def factor(Hdev, n, precision="fp64", structure=None, n_positive=None, rebuild=None, order=None):
+def factor(Hdev, n, precision="fp64", structure=None, n_positive=None, rebuild=None, order=None,
+           keep=False):
     """Factor a device HeadMat (triangles-first order).  precision 'fp64'
     factors in place; 'mixed' keeps Hdev as the FP64 residual operator and
     factors an FP32 copy; 'mixed16' does the same with split-FP16 MFMA
@@ -746,14 +749,19 @@ def factor(Hdev, n, precision="fp64", structure=None, n_positive=None, rebuild=N
     matrix is factored by LU with partial pivoting (the reference's DSPTRF
     pivots too, symmatrix.cpp:133-152): for the mixed paths Hdev itself,
     which is intact; for 'fp64', whose failed factorisation overwrote Hdev,
-    the matrix rebuild() returns (else OpenMEEGError)."""
+    the matrix rebuild() returns (else OpenMEEGError).
+
+    keep: Hdev stays intact on every path; what would run in place, the
+    fallbacks of a later solve() among it, runs on a copy (rebuild is not
+    needed)."""
     torch = _t()
+    own = (lambda: Hdev.clone()) if keep else (lambda: Hdev)
     if precision == "fp64_lu":
-        return _lu_factor(Hdev, n)
+        return _lu_factor(own(), n)
     if order is not None and structure is None:
         raise ValueError("a factor order needs the block structure")
-    if order is not None and precision == "fp64" and not _room_for(8 * n * n):
-        order = None
+    if order is not None and precision == "fp64" and not keep and not _room_for(8 * n * n):
+        order = None   # (with keep, a copy is needed in either order)
     info = C.c_int32()
     sargs = _block_args(structure)
     blocks = sargs[2:] if sargs else ()
@@ -769,31 +777,32 @@ def factor(Hdev, n, precision="fp64", structure=None, n_positive=None, rebuild=N
             check(lib().omh_sym_reorder(_ptr(Hdev), n, _ptr(L), n, 8, n, blocks[0], blocks[1], optr, _stream()))
             check(lib().omh_sym_factor_f64_blocks(_ptr(L), n, n, _ptr(work), *fblocks, C.byref(info), _stream()))
         elif blocks:
-            L = Hdev
-            check(lib().omh_sym_factor_f64_blocks(_ptr(Hdev), n, n, _ptr(work), *blocks, C.byref(info), _stream()))
+            L = own()
+            check(lib().omh_sym_factor_f64_blocks(_ptr(L), n, n, _ptr(work), *blocks, C.byref(info), _stream()))
         else:
-            L = Hdev
-            check(lib().omh_sym_factor_f64(_ptr(Hdev), n, n, _ptr(work), C.byref(info), _stream()))
-        F = Factor(L, n, work, "fp64", structure=structure, n_positive=n_positive, order=order)
+            L = own()
+            check(lib().omh_sym_factor_f64(_ptr(L), n, n, _ptr(work), C.byref(info), _stream()))
+        F = Factor(L, n, work, "fp64", structure=structure, n_positive=n_positive, order=order, keep=keep)
         elem = 8
     elif precision in ("mixed", "mixed16"):
         # the reordered copy's columns start on 16 bytes: vector loads in the
         # panels, and the split products of the solves
         ld = n if order is None else (n + 3) // 4 * 4
-        L32 = torch.empty(ld * n, dtype=torch.float32, device="cuda")
+        L = torch.empty(ld * n, dtype=torch.float32, device="cuda")
         if order is not None:
-            check(lib().omh_sym_reorder(_ptr(Hdev), n, _ptr(L32), ld, 4, n, blocks[0], blocks[1], optr, _stream()))
+            check(lib().omh_sym_reorder(_ptr(Hdev), n, _ptr(L), ld, 4, n, blocks[0], blocks[1], optr, _stream()))
         else:
-            check(lib().omh_convert_f64_f32(_ptr(Hdev), n, _ptr(L32), n, n, n, 1, _stream()))
+            check(lib().omh_convert_f64_f32(_ptr(Hdev), n, _ptr(L), n, n, n, 1, _stream()))
         work = torch.empty(int(lib().omh_factor_workspace_bytes(n, 4)), dtype=torch.uint8, device="cuda")
         if blocks:
             fn = lib().omh_sym_factor_f32_blocks if precision == "mixed" else lib().omh_sym_factor_f32_split_blocks
-            check(fn(_ptr(L32), n, ld, _ptr(work), *(fblocks if order is not None else blocks), C.byref(info),
+            check(fn(_ptr(L), n, ld, _ptr(work), *(fblocks if order is not None else blocks), C.byref(info),
                      _stream()))
         else:
             fn = lib().omh_sym_factor_f32 if precision == "mixed" else lib().omh_sym_factor_f32_split
-            check(fn(_ptr(L32), n, n, _ptr(work), C.byref(info), _stream()))
-        F = Factor(L32, n, work, "mixed", H64=Hdev, structure=structure, n_positive=n_positive, order=order, ld=ld)
+            check(fn(_ptr(L), n, n, _ptr(work), C.byref(info), _stream()))
+        F = Factor(L, n, work, "mixed", H64=Hdev, structure=structure, n_positive=n_positive, order=order, ld=ld,
+                   keep=keep)
         elem = 4
     else:
         raise ValueError("precision must be 'fp64', 'mixed', 'mixed16' or 'fp64_lu'")
@@ -812,17 +821,17 @@ def factor(Hdev, n, precision="fp64", structure=None, n_positive=None, rebuild=N
             reason = "pivot sign at unknown %d" % first.value
     if reason is None:
         return F
-    del F
+    del F, L, work
     if order is not None:
         # Hdev is intact: the factorisation in its own order
-        F = factor(Hdev, n, precision, structure, n_positive, rebuild)
+        F = factor(Hdev, n, precision, structure, n_positive, rebuild, keep=keep)
         F.reorder_breakdown = reason
         return F
-    if precision == "fp64":
+    if precision == "fp64" and not keep:
         if rebuild is None:
             raise _lib.OpenMEEGError("pivot-free factorisation broke down (%s)" % reason)
         Hdev = rebuild()
-    F = _lu_factor(Hdev, n)
+    F = _lu_factor(own(), n)
     F.breakdown = reason
     return F
 
@@ -833,19 +842,20 @@ def factor(Hdev, n, precision="fp64", structure=None, n_positive=None, rebuild=N
 HEADMAT_FAR_FIELD = 1
 
 
-def _head_factor(geom, H, precision, integrator=None, far_field=False):
+def _head_factor(geom, H, precision, integrator=None, far_field=False, keep=False):
     """factor() of a pipeline's HeadMat H with the geometry's block
     structure, its mesh-by-mesh factor order (Geometry.factor_order; the
     environment variable OMH_FACTOR_ORDER=0 keeps the triangles-first order)
     and pivot-sign pattern (triangle unknowns +); an FP64 breakdown
-    re-assembles H for the pivoted LU."""
+    re-assembles H for the pivoted LU (keep: H stays intact and the LU takes
+    a copy)."""
     n = geom.size
     structure = geom.factor_segments()
     order = None
     if structure is not None and os.environ.get("OMH_FACTOR_ORDER", "1") != "0":
         order = geom.factor_order()
     return factor(H, n, precision, structure=structure, n_positive=n - geom.n_vertex_unknowns,
-                  rebuild=lambda: _head_mat_device(geom, integrator, far_field), order=order)
+                  rebuild=lambda: _head_mat_device(geom, integrator, far_field), order=order, keep=keep)
 
 
 def _head_mat_device(geom, integrator=None, far_field=False):

@@ -31,7 +31,7 @@ import numpy as np
 
 from . import _lib
 from ._lib import check, lib, ORDER_TRIANGLES_FIRST
-from .api import (Head2EEGMat, Integrator, _dev_f64, _eeg_rhs, _head_mat_device, _ptr, _stream, _t, factor)
+from .api import (Head2EEGMat, Integrator, _dev_f64, _eeg_rhs, _head_mat_device, _head_factor, _ptr, _stream, _t)
 
 
 def _gemm(ta, tb, m, n, k, A, lda, B, ldb, Cout, ldc, a_off=0, b_off=0, alpha=1.0, beta=0.0):
@@ -123,20 +123,16 @@ class EEGForward:
         doms = (C.c_int32 * max(nd, 1))()
         check(lib().omh_locate_domains(g._h, _ptr(dip), 6, nd, doms, _stream()))
         H = _head_mat_device(g, Integrator(self.order), far_field=self.precision != "fp64")
-        Hkeep = H.clone() if self.precision == "fp64" else H   # the FP64 factor overwrites H
         D = _dev_f64(n * max(nd, 1))
         check(lib().omh_dip_source_mat(g._h, _ptr(dip), nd, doms, self.order, 0, 0.0, _ptr(D), n,
                                        ORDER_TRIANGLES_FIRST, _stream()))
-        # the pipelines' block structure and mesh-by-mesh order: the factor and
-        # the solves skip the blocks that are zero
-        structure = g.factor_segments()
-        F = factor(H, n, self.precision, structure=structure,
-                   order=g.factor_order() if structure is not None else None)
+        # the backward pass reads H: it stays intact beside its factor
+        F = _head_factor(g, H, self.precision, keep=True)
         Y = self._E.clone()
         F.solve(Y, ne, max_iter=self.max_refine, tol=self.refine_tol)
         G = _dev_f64(ne * max(nd, 1))
         _gemm(1, 0, ne, nd, n, Y, n, D, n, G, ne)
-        state = dict(H=Hkeep, F=F, Y=Y, D=D, dip=dip, doms=doms, sigma=self._sigma.copy(), nd=nd)
+        state = dict(H=H, F=F, Y=Y, D=D, dip=dip, doms=doms, sigma=self._sigma.copy(), nd=nd)
         return G[: ne * nd].view(nd, ne).t().contiguous(), state
 
     def _backward(self, st, gout, need_dip, need_sigma):

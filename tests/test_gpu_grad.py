@@ -132,6 +132,41 @@ def test_moved_conductivity_gradient(setup):
         assert abs(gs[d] - fd) < 1e-6 * np.abs(gs).max()
 
 
+@pytest.mark.parametrize("precision", ["fp64", "mixed", "mixed16"])
+def test_breakdown_keeps_the_gradients(setup, monkeypatch, precision):
+    """A factorisation that breaks down (every unknown declared positive, so
+    that each vertex pivot's sign contradicts) goes to the matrix's own order
+    and then to the pivoted LU, and one whose refinement stops too early to
+    its FP64 factor; the HeadMat of the conductivity gradient stays intact:
+    gains to 1e-9, gradients to 1e-6 of the undisturbed ones (as for mixed
+    against FP64 above; 1e-9 with FP64 throughout)."""
+    om, meshes, dip, el, _, R = setup
+    from openmeeg_amd import api
+    g = om.make_nested_geometry(meshes, LAYERS[1])
+    ref = _loss_and_grads(om.EEGForward(g, el, precision="fp64"), dip, R)
+
+    def check(model, tol):
+        got = _loss_and_grads(model, dip, R)
+        dG = float((got[4] - ref[4]).detach().norm() / ref[4].detach().norm())
+        errs = [np.linalg.norm(x - y) / np.linalg.norm(y) for x, y in zip(got[1:4], ref[1:4])]
+        print("%s: gain %.3e, gradients %s" % (precision, dG, errs), flush=True)
+        assert dG < 1e-9 and max(errs) < tol
+
+    tol = 1e-9 if precision == "fp64" else 1e-6
+    if precision != "fp64":
+        check(om.EEGForward(g, el, precision=precision, max_refine=1), tol)
+    seen, real = [], api.factor
+
+    def all_positive(H, n, precision="fp64", structure=None, n_positive=None, *a, **kw):
+        F = real(H, n, precision, structure, n if n_positive is not None else None, *a, **kw)
+        seen.append(F)
+        return F
+
+    monkeypatch.setattr(api, "factor", all_positive)
+    check(om.EEGForward(g, el, precision=precision), tol)
+    assert seen and seen[-1].pivoted and seen[-1].reorder_breakdown.startswith("pivot sign")
+
+
 def test_c3_fit_gradient_matches_fd(setup):
     """The 128-electrode, 4096-dipole fit on the 2562-vertex 3-layer head:
     L = 0.5 |G(p, q, sigma) - T|^2 with targets T at SNR 10, from a start
