@@ -49,8 +49,7 @@ enum ScratchSlot {
     SCR_RESID_XT = 9,  // the refinement's transposed solution (structured residual products)
     SCR_ROWMAP = 10,   // row map of a reordered factor (segment order)
     SCR_SOLVE_SCALES = 11,   // the refinement's cache of the split solve products' scales
-    SCR_SOLVE_TMP = 12,      // one block of rows of a wide FP64 solve
-    SCR_NSLOTS = 13
+    SCR_NSLOTS = 12
 };
 void* scratch(ScratchSlot slot, size_t bytes, hipStream_t st);
 void release_scratch();

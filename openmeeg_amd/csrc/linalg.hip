@@ -3543,6 +3543,97 @@ __global__ void __launch_bounds__(SG_THREADS) k_solve_pair(const T* __restrict__
     }
 }
 
+// W_b <- Linv_b W_b (BACK: Linv_b^T W_b) in place for many FP64 right-hand
+// sides: a workgroup holds BS_COLS columns of the block's nb rows of W in
+// LDS, so that it alone reads and writes them; each of its 8 waves forms 32
+// rows with MFMAs.  Bound by MFMA issue (8 x 64 steps of four 16 x 16 x 4
+// products a wave).  It needs no memory besides W, so that solves from
+// several threads and streams share nothing.  8136 right-hand sides: 28 us a
+// block (a GEMM into a buffer and a copy back: 45 us).  Linv beyond nb is not
+// read as a number: rows there are not stored, columns there are cleared.
+constexpr int BS_THREADS = 512, BS_COLS = 32;
+
+template <bool BACK>
+__global__ void __launch_bounds__(BS_THREADS) k_block_solve(const double* __restrict__ Linv, int nb,
+                                                            double* __restrict__ W, int64_t ldw, int64_t r) {
+    constexpr int NB = FACT_NB;
+    static_assert(NB == 32 * (BS_THREADS / 64) && BS_THREADS == 2 * NB, "a wave takes 32 rows, two threads a row");
+    __shared__ double Ws[BS_COLS][NB + 2];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t c0 = (int64_t)blockIdx.x * BS_COLS;
+    const int nc = (int)min<int64_t>(BS_COLS, r - c0);
+    const int wi = tid % NB, wc = tid / NB;   // the thread's row and columns wc, wc + 2, .. of the strip
+    if (wi < nb) {
+#pragma unroll
+        for (int c = 0; c < BS_COLS; c += 2) Ws[wc + c][wi] = W[wi + (c0 + min(wc + c, nc - 1)) * ldw];
+    } else {
+#pragma unroll
+        for (int c = 0; c < BS_COLS; c += 2) Ws[wc + c][wi] = 0.0;
+    }
+    __syncthreads();
+    const int li = lane & 15, q = lane >> 4;
+    // 16 columns of op(Linv) at a time: a[t][s] is row 32 wave + 16 t + li,
+    // column k0 + kq + ks s, the columns of a product lying along memory: one
+    // of each four (forward), four side by side in 16-byte loads (backward)
+    constexpr int ks = BACK ? 1 : 4;
+    const int kq = BACK ? 4 * q : q;
+    typedef double pair_t __attribute__((ext_vector_type(2), aligned(8)));   // the workspace may lie on 8 bytes
+    auto load = [&](int k0, double (&a)[2][4]) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int row = 32 * wave + 16 * t + li, k = k0 + kq;
+            if (BACK) {
+                const pair_t* p = reinterpret_cast<const pair_t*>(Linv + k + row * NB);
+                const pair_t x = p[0], y = p[1];
+                a[t][0] = x.x; a[t][1] = x.y; a[t][2] = y.x; a[t][3] = y.y;
+            } else {
+#pragma unroll
+                for (int s = 0; s < 4; ++s) a[t][s] = Linv[row + (k + ks * s) * NB];
+            }
+        }
+        if (k0 + 16 > nb) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                if (k0 + kq + ks * s >= nb) a[0][s] = a[1][s] = 0.0;
+        }
+    };
+    double4_t acc[2][2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) acc[t][b] = double4_t{0.0, 0.0, 0.0, 0.0};
+    double a[2][4], an[2][4];
+    load(0, a);
+    for (int k0 = 0; k0 < nb; k0 += 16) {
+        load(min(k0 + 16, NB - 16), an);   // past the end: unused
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                const double x = Ws[16 * b + li][k0 + kq + ks * s];
+#pragma unroll
+                for (int t = 0; t < 2; ++t) acc[t][b] = Acc<double>::mfma(a[t][s], x, acc[t][b]);
+            }
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) a[t][s] = an[t][s];
+    }
+    __syncthreads();   // the strip has been read
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) Ws[16 * b + li][32 * wave + 16 * t + Acc<double>::row(lane, e)] = acc[t][b][e];
+    __syncthreads();
+    if (wi < nb) {
+#pragma unroll
+        for (int c = 0; c < BS_COLS; c += 2)
+            if (wc + c < nc) W[wi + (c0 + wc + c) * ldw] = Ws[wc + c][wi];
+    }
+}
+
 // Row intervals [start, start + len) of a split solve product, cut into
 // tiles of `tile` rows: tile x lies in the interval k with tile0[k] <= x <
 // tile0[k + 1].
@@ -3896,16 +3987,9 @@ static void sym_solve_impl(const T* L, int64_t n, int64_t lda, const void* work,
         return cdiv(rows, 64) * cdiv(r, 64) >= 1024;
     };
     // strips of 2 right-hand sides up to 1024 of them (128 workgroups for
-    // 256; 8-wide strips took twice as long per group at 256); beyond, GEMMs
-    // (FP64) or strips of 8
+    // 256; 8-wide strips took twice as long per group at 256); beyond, block
+    // products and GEMMs (FP64) or strips of 8
     const bool narrow = r <= 1024;
-    T* tmp = nullptr;   // a block of rows of W (not under capture: the scratch may have to grow)
-    if (!narrow && sizeof(T) == 8) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        OMH_HIP(hipStreamIsCapturing(st, &cap));
-        if (cap == hipStreamCaptureStatusNone)
-            tmp = (T*)scratch(SCR_SOLVE_TMP, sizeof(T) * (size_t)FACT_NB * (size_t)r, st);
-    }
     auto group_solve = [&](bool back, int64_t k0, int64_t gend, bool split) {
         WSplit ws;
         if (split) ws = sb->ws;
@@ -3919,18 +4003,20 @@ static void sym_solve_impl(const T* L, int64_t n, int64_t lda, const void* work,
             const unsigned g = (unsigned)cdiv(r, 2);
             if (back) k_solve_group<T, true, 2><<<g, 256, 0, st>>>(L, lda, Dinv, k0, gend, W, ldw, r, ws);
             else k_solve_group<T, false, 2><<<g, 256, 0, st>>>(L, lda, Dinv, k0, gend, W, ldw, r, ws);
-        } else if (tmp) {
+        } else if constexpr (sizeof(T) == 8) {
             // more right-hand sides than strips can use: the same block
-            // products as whole GEMMs (8136 unknowns, as many right-hand
-            // sides: about 0.3 ms a group against 1.17 ms forward and 0.52 ms
-            // backward for strips of 8, which read L for each strip)
+            // products, the diagonal ones in place and the others as whole
+            // GEMMs (8136 unknowns, as many right-hand sides: 0.31 ms a group
+            // against 1.17 ms forward and 0.52 ms backward for strips of 8,
+            // which read L for each strip)
             const int nbk = (int)cdiv(gend - k0, FACT_NB);
             for (int bi = 0; bi < nbk; ++bi) {
                 const int64_t kb = k0 + (int64_t)(back ? nbk - 1 - bi : bi) * FACT_NB;
-                const int64_t nb = std::min<int64_t>(FACT_NB, gend - kb);
-                gemm<T>(back, false, false, nb, r, nb, T(1), Dinv + (size_t)(kb / FACT_NB) * FACT_NB * FACT_NB, FACT_NB,
-                        W + kb, ldw, T(0), tmp, FACT_NB, st);
-                k_copy<T><<<grid_for(nb * r), 256, 0, st>>>(tmp, FACT_NB, W + kb, ldw, nb, r);
+                const int nb = (int)std::min<int64_t>(FACT_NB, gend - kb);
+                const T* Li = Dinv + (size_t)(kb / FACT_NB) * FACT_NB * FACT_NB;
+                const unsigned g = (unsigned)cdiv(r, BS_COLS);
+                if (back) k_block_solve<true><<<g, BS_THREADS, 0, st>>>(Li, nb, W + kb, ldw, r);
+                else k_block_solve<false><<<g, BS_THREADS, 0, st>>>(Li, nb, W + kb, ldw, r);
                 OMH_LAUNCH_CHECK();
                 if (back && kb > k0)
                     gemm<T>(true, false, false, kb - k0, r, nb, T(-1), L + kb + k0 * lda, lda, W + kb, ldw, T(1),

@@ -1,8 +1,11 @@
 """Triangular solves of the stored factor over the paths a group of four
 256-blocks can take: whole groups (k_solve_pair), partial groups and odd
-leading dimensions (k_solve_group), more than 1024 right-hand sides (block
-GEMMs for FP64); FP32 split products and their scale cache."""
+leading dimensions (k_solve_group), more than 1024 right-hand sides (FP64:
+diagonal blocks in place and GEMMs, the same under capture and beside other
+threads' solves); FP32 split products and their scale cache."""
 import ctypes as C
+import threading
+import time
 
 import numpy as np
 import pytest
@@ -55,6 +58,117 @@ def test_solve_residual(om, n, r, pad, dtype):
     assert float(res.max()) < 10 * np.sqrt(n) * np.finfo(dtype).eps
     if pad:
         assert torch.equal(dB[:, n:].double(), B0[:, n:])
+
+
+def _system(n, r, seed, pad=0):
+    """A factored quasi-definite FP64 matrix and its right-hand sides."""
+    import torch
+    from openmeeg_amd import _lib
+    lib = _lib.lib()
+    rng = np.random.default_rng(seed)
+    A = rng.standard_normal((n, n)) / np.sqrt(n)
+    A = 0.25 * (A + A.T) + np.diag(np.where(np.arange(n) < n // 2, 2.0, -2.0))
+    dA = torch.zeros((n, n + pad), dtype=torch.float64, device="cuda")
+    dA[:, :n] = torch.from_numpy(A)
+    work = torch.zeros(int(lib.omh_factor_workspace_bytes(n, 8)), dtype=torch.uint8, device="cuda")
+    info = C.c_int32()
+    _lib.check(lib.omh_sym_factor_f64(C.c_void_p(dA.data_ptr()), n, n + pad, C.c_void_p(work.data_ptr()),
+                                      C.byref(info), C.c_void_p(0)))
+    assert info.value == 0
+    B = torch.from_numpy(rng.standard_normal((r, n))).cuda()
+
+    def solve(X, stream):
+        _lib.check(lib.omh_sym_solve_f64(C.c_void_p(dA.data_ptr()), n, n + pad, C.c_void_p(work.data_ptr()),
+                                         C.c_void_p(X.data_ptr()), n, r, C.c_void_p(stream.cuda_stream)))
+
+    torch.cuda.synchronize()
+    return B, solve
+
+
+@pytest.mark.parametrize("n,r,pad", [(1024, 1025, 0), (1300, 1100, 1), (2309, 2000, 3)])
+def test_many_rhs_same_under_capture(om, n, r, pad):
+    """A captured FP64 solve of more than 1024 right-hand sides takes the
+    eager call's kernels: the same bits on every replay."""
+    import torch
+    B, solve = _system(n, r, n, pad)
+    X, Y = B.clone(), B.clone()
+    solve(X, torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        solve(Y, torch.cuda.current_stream())
+    for _ in range(3):
+        Y.copy_(B)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(X, Y)
+
+
+def test_many_rhs_on_two_streams(om):
+    """FP64 solves of more than 1024 right-hand sides on two streams share
+    nothing: the second one runs while the first stream is still busy."""
+    import torch
+    n, r = 1300, 1100
+    B, solve = _system(n, r, 5)
+    streams = [torch.cuda.Stream() for _ in range(8)]
+    X = [B.clone() for _ in streams]
+    torch.cuda.synchronize()
+    for x, s in zip(X, streams):
+        solve(x, s)
+        s.synchronize()
+    busy, done = streams[0], torch.cuda.Event()
+    solve(X[0], busy)
+    with torch.cuda.stream(busy):
+        torch.cuda._sleep(int(1e9))
+        done.record()
+    # a stream that does not share the first one's hardware queue
+    for x, s in zip(X[1:], streams[1:]):
+        mark = torch.cuda.Event()
+        with torch.cuda.stream(s):
+            x.copy_(B)
+            mark.record()
+        t = time.time()
+        while not mark.query() and time.time() - t < 0.02:
+            pass
+        if mark.query():
+            break
+    assert mark.query() and not done.query(), "no stream runs beside the busy one"
+    solve(x, s)
+    s.synchronize()
+    assert not done.query()
+    torch.cuda.synchronize()
+
+
+def test_many_rhs_from_several_threads(om):
+    """FP64 solves of more than 1024 right-hand sides hold no buffer that
+    calls share: three host threads with factors and streams of their own
+    get the bits of the solves one after the other."""
+    import torch
+    systems = [_system(n, r, n + r) for n, r in ((1536, 1500), (1300, 1100), (2048, 1030))]
+    want = []
+    for B, solve in systems:
+        X = B.clone()
+        solve(X, torch.cuda.current_stream())
+        want.append(X)
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(k):
+        B, solve = systems[k]
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for _ in range(20):
+                X = B.clone()
+                solve(X, stream)
+                if not torch.equal(X, want[k]):
+                    bad.append(k)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(len(systems))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
 
 
 def test_split_products_scale_cache_many_rhs(om, monkeypatch):
