@@ -49,7 +49,8 @@ enum ScratchSlot {
     SCR_RESID_XT = 9,  // the refinement's transposed solution (structured residual products)
     SCR_ROWMAP = 10,   // row map of a reordered factor (segment order)
     SCR_SOLVE_SCALES = 11,   // the refinement's cache of the split solve products' scales
-    SCR_NSLOTS = 12
+    SCR_RESID_PART = 12,     // its chunks' partial sums (not SCR_GEMM: a GEMM on another thread may run beside it)
+    SCR_NSLOTS = 13
 };
 void* scratch(ScratchSlot slot, size_t bytes, hipStream_t st);
 void release_scratch();

@@ -4288,8 +4288,9 @@ static void residual_update(const double* H, int64_t n, int64_t ldh, const doubl
     // on the products go whole.
     const int64_t tiles = cdiv(n, 64) * cdiv(r, 64);
     const int nsplit = (int)std::max<int64_t>(1, std::min<int64_t>(8, 1280 / std::max<int64_t>(tiles, 1)));
-    double* W = nsplit > 1 ? (double*)scratch(SCR_GEMM, sizeof(double) * (size_t)nsplit * (size_t)n * (size_t)r, st)
-                           : nullptr;
+    double* W = nsplit > 1
+                    ? (double*)scratch(SCR_RESID_PART, sizeof(double) * (size_t)nsplit * (size_t)n * (size_t)r, st)
+                    : nullptr;
     SidePool& sp = side_pool();
     OMH_HIP(hipEventRecord(sp.fork, st));
     for (int i = 0; i < N_SIDE; ++i) OMH_HIP(hipStreamWaitEvent(sp.s[i], sp.fork, 0));

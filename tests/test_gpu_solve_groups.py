@@ -171,6 +171,55 @@ def test_many_rhs_from_several_threads(om):
     assert not bad
 
 
+def test_refinement_beside_a_split_gemm(om):
+    """The chunked residual of a small head's refinement and the split-K
+    products of omh_gemm_f64 on another thread use buffers of their own: the
+    bits of each alone."""
+    import torch
+    from openmeeg_amd import _lib, spheres as S
+    from openmeeg_amd.api import _head_mat_device, factor
+    g = om.make_nested_geometry(S.nested_sphere_meshes(8, (0.87, 0.92, 1.0)), (1.0, 0.0125, 1.0))
+    n, r = g.size, 37
+    H = _head_mat_device(g, far_field=True)
+    F = factor(H, n, "mixed", structure=g.factor_segments(), order=g.factor_order())
+    rng = np.random.default_rng(1)
+    B = torch.from_numpy(rng.standard_normal(n * r)).cuda()
+    m, q, k = 96, 320, 20000
+    P = torch.from_numpy(rng.standard_normal(m * k)).cuda()
+    Q = torch.from_numpy(rng.standard_normal(q * k)).cuda()
+
+    def refine(stream):
+        X = B.clone()
+        F.solve(X, r, tol=1e-12)
+        return X
+
+    def gemm(stream):
+        Z = torch.empty(m * q, dtype=torch.float64, device="cuda")
+        _lib.check(_lib.lib().omh_gemm_f64(1, 0, m, q, k, 1.0, C.c_void_p(P.data_ptr()), k, C.c_void_p(Q.data_ptr()), k,
+                                           0.0, C.c_void_p(Z.data_ptr()), m, C.c_void_p(stream.cuda_stream)))
+        return Z
+
+    calls = (refine, gemm)
+    want = [f(torch.cuda.current_stream()) for f in calls]
+    assert F.iterations >= 2
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(i):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for _ in range(30):
+                if not torch.equal(calls[i](stream), want[i]):
+                    bad.append(calls[i].__name__)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(calls))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+
+
 def test_split_products_scale_cache_many_rhs(om, monkeypatch):
     """Enough right-hand sides that the split products run (1024 tiles of
     64 x 64 and more): cached scales against scales formed by every solve,
