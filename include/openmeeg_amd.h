@@ -441,8 +441,12 @@ int omh_permute_rows(const double* d_src, int64_t lds, double* d_dst, int64_t ld
 /* Kernel timing for benchmarks (no reference counterpart): when enabled,
  * HIP event pairs are recorded on the launch stream around the named
  * kernels: "factor_update_f32_t128", "factor_update_f32_t64",
- * "factor_update_f64_t64" (interior launches of the trailing-update GEMM
- * with 128- or 64-wide tiles), "diag_factor_f64", "diag_factor_f32",
+ * "factor_update_f64_t64", "factor_update_f64_t128" (the trailing-update
+ * GEMM with 128- or 64-wide tiles; FP64 128: its whole tiles),
+ * "factor_update_f32s" (split-FP16 update), "diag_factor_f64",
+ * "diag_factor_f32", "solve_update_f32s" (split-FP16 solve products),
+ * "residual_f64_t128", "residual_f64_split" (the refinement's residual
+ * products on 128-wide tiles or in chunks of the inner dimension),
  * "s_block", "d_pairs".  omh_profile_enable clears the
  * records; omh_profile_read returns the launches, the summed seconds and the
  * summed algorithmic work (flop for the factor kernels, Gauss-point

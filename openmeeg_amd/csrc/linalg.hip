@@ -4329,11 +4329,13 @@ static void residual_update(const double* H, int64_t n, int64_t ldh, const doubl
             if (nsplit > 1 && kc >= 256 && kc < k) {
                 double* Wp = W + (size_t)nsplit * r0 * r;   // the segment's own part: the segments run concurrently
                 const int ns2 = (int)cdiv(k, kc);
+                ProfScope ps("residual_f64_split", 2.0 * (double)m * (double)r * (double)k, ss);
                 splitk_tiles<double, false, true>(aligned_for_vec(Hs, ldh) && aligned_for_vec(Xs, r), m, r, k, kc, ns2,
                                                   Hs, ldh, Xs, r, Wp, ss);
                 k_splitk_sum<double><<<grid_for(m * r), 256, 0, ss>>>(Wp, ns2, m, r, -1.0, 1.0, R + r0, ldr);
                 OMH_LAUNCH_CHECK();
-            } else if (!gemm_f64_dma(false, m, r, k, -1.0, Hs, ldh, Xs, r, 1.0, R + r0, ldr, ss, nullptr, 64, true)) {
+            } else if (!gemm_f64_dma(false, m, r, k, -1.0, Hs, ldh, Xs, r, 1.0, R + r0, ldr, ss, "residual_f64", 64,
+                                     true)) {
                 gemm<double>(false, true, false, m, r, k, -1.0, Hs, ldh, Xs, r, 1.0, R + r0, ldr, ss);
             }
             t = u;

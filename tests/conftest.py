@@ -22,6 +22,28 @@ def rel_fro(a, b):
     return float(np.linalg.norm(a - b) / np.linalg.norm(b))
 
 
+class Launches:
+    """Counts the library's timed launches inside the block: a test of one of
+    several kernels shows with it that the kernel ran."""
+
+    def __enter__(self):
+        from openmeeg_amd import _lib
+        _lib.check(_lib.lib().omh_profile_enable(1))
+        return self
+
+    def __call__(self, name):
+        import ctypes as C
+        from openmeeg_amd import _lib
+        calls, sec, work = C.c_int64(), C.c_double(), C.c_double()
+        _lib.check(_lib.lib().omh_profile_read(name.encode(), C.byref(calls), C.byref(sec), C.byref(work)))
+        return calls.value
+
+    def __exit__(self, *exc):
+        from openmeeg_amd import _lib
+        _lib.check(_lib.lib().omh_profile_enable(0))
+        return False
+
+
 @pytest.fixture(scope="session")
 def golden():
     return GOLDEN

@@ -14,7 +14,7 @@ import os
 import numpy as np
 import pytest
 
-from conftest import GOLDEN, rel_fro
+from conftest import GOLDEN, Launches, rel_fro
 
 pytestmark = pytest.mark.gpu
 
@@ -319,15 +319,22 @@ def test_fp64_factor_dma_tiles_bitwise(om, monkeypatch):
         assert torch.equal(L["dma"], L["tiles64"])
         del L
     Hf = _head_mat_device(g, far_field=True)
-    B = torch.from_numpy(np.random.default_rng(3).standard_normal(n * 64)).cuda()
+    # from 641 tiles of 64 x 64 on the residual's products go whole (not in
+    # chunks); four tile columns of 128 give the vertex segments (21 tile
+    # rows, the last one partial) the 64 tiles the DMA kernel asks for
+    r = 512
+    B = torch.from_numpy(np.random.default_rng(3).standard_normal(n * r)).cuda()
     F = factor(Hf, n, "mixed16", structure=g.factor_segments())
     X = {}
     for mode in ("dma", "tiles64"):
         if mode == "tiles64":
             monkeypatch.setenv("OMH_GEMM_F64_DMA", "0")
         X[mode] = B.clone()
-        F.solve(X[mode], 64, max_iter=10, tol=1e-10)
-        torch.cuda.synchronize()
+        with Launches() as ran:
+            F.solve(X[mode], r, max_iter=10, tol=1e-10)
+            torch.cuda.synchronize()
+            tiles, chunks = ran("residual_f64_t128"), ran("residual_f64_split")
+        assert chunks == 0 and (tiles > 0) == (mode == "dma")
         monkeypatch.delenv("OMH_GEMM_F64_DMA", raising=False)
     print("refined solution max |diff| %.3e after %d iterations" % (float((X["dma"] - X["tiles64"]).abs().max()),
                                                                     F.iterations), flush=True)
@@ -643,34 +650,43 @@ def test_split_solve_products(om):
     solution: the split solve's error is at most 4x the FP32 solve's (plus
     1e-7), and the refined solution's residual is < 1e-12.  3 layers of 2562
     vertices (n = 17926: 17 full groups and a partial one, whose products
-    stay FP32) and 200 right-hand sides (a full and a partial 128-column
-    tile)."""
+    stay FP32), leading dimension 17928 (the split products read 16-byte
+    aligned columns) and 600 right-hand sides (two full and a partial
+    256-column tile; more than 6500 rows give the 1024 tiles of 64 x 64 from
+    which the split products run)."""
     import ctypes as C
     import torch
     from openmeeg_amd import spheres as S, _lib
-    from openmeeg_amd.api import _head_mat_device, factor
+    from openmeeg_amd.api import _head_mat_device
     g = om.make_nested_geometry(S.nested_sphere_meshes(16, (0.87, 0.92, 1.0)), (1.0, 0.0125, 1.0))
-    n, r = g.size, 200
+    n, r = g.size, 600
     H = _head_mat_device(g, far_field=True)
-    F = factor(H, n, "mixed16")
+    p = lambda t: C.c_void_p(t.data_ptr())
+    lib, ld = _lib.lib(), (n + 3) // 4 * 4
+    L = torch.empty(ld * n, dtype=torch.float32, device="cuda")
+    work = torch.empty(int(lib.omh_factor_workspace_bytes(n, 4)), dtype=torch.uint8, device="cuda")
+    info = C.c_int32()
+    _lib.check(lib.omh_convert_f64_f32(p(H), n, p(L), ld, n, n, 1, C.c_void_p(0)))
+    _lib.check(lib.omh_sym_factor_f32_split(p(L), n, ld, p(work), C.byref(info), C.c_void_p(0)))
+    assert info.value == 0
     B = torch.from_numpy(np.random.default_rng(21).standard_normal(n * r)).cuda()
 
     def mixed(max_iter, tol):
         X = torch.full((n * r,), np.nan, dtype=torch.float64, device="cuda")
         it, rel = C.c_int32(), C.c_double()
-        rc = _lib.lib().omh_mixed_solve(C.c_void_p(H.data_ptr()), n, n, C.c_void_p(F.L.data_ptr()), n,
-                                        C.c_void_p(F.work.data_ptr()), C.c_void_p(B.data_ptr()), n,
-                                        C.c_void_p(X.data_ptr()), n, r, max_iter, tol, C.byref(it), C.byref(rel),
-                                        C.c_void_p(0))
-        assert rc in (0, _lib.STATUS_NOT_CONVERGED), _lib.lib().omh_last_error()
+        rc = lib.omh_mixed_solve(p(H), n, n, p(L), ld, p(work), p(B), n, p(X), n, r, max_iter, tol, C.byref(it),
+                                 C.byref(rel), C.c_void_p(0))
+        assert rc in (0, _lib.STATUS_NOT_CONVERGED), lib.omh_last_error()
         return X, rc, it.value
 
-    X1, rc1, it1 = mixed(1, 1e-12)          # one split solve, then stop
+    with Launches() as ran:
+        X1, rc1, it1 = mixed(1, 1e-12)          # one split solve, then stop
+        split = ran("solve_update_f32s")
+    assert split >= 20                       # of the 17 groups' products forward and backward
     Xr, rcr, itr = mixed(10, 1e-12)          # refined
     assert rc1 == _lib.STATUS_NOT_CONVERGED and rcr == 0
     W = B.to(torch.float32).clone()
-    _lib.check(_lib.lib().omh_sym_solve_f32(C.c_void_p(F.L.data_ptr()), n, n, C.c_void_p(F.work.data_ptr()),
-                                            C.c_void_p(W.data_ptr()), n, r, C.c_void_p(0)))
+    _lib.check(lib.omh_sym_solve_f32(p(L), n, ld, p(work), p(W), n, r, C.c_void_p(0)))
     torch.cuda.synchronize()
     nr = torch.linalg.norm(Xr)
     e_split = float(torch.linalg.norm(X1 - Xr) / nr)
@@ -889,7 +905,9 @@ def test_refinement_scale_cache_bitwise(om, monkeypatch):
     scales the first one formed (they depend on the factor only): the
     refined solution is bitwise the one that forms them in every solve.  4
     layers of 1442 vertices (n = 14408), mesh-by-mesh factor order, block
-    structure."""
+    structure; 640 right-hand sides, so that groups that reach two meshes
+    (more than 6500 rows) have the 1024 tiles of 64 x 64 from which the split
+    products run."""
     import torch
     from openmeeg_amd.api import _head_mat_device, factor
     from openmeeg_amd import spheres as S
@@ -898,14 +916,17 @@ def test_refinement_scale_cache_bitwise(om, monkeypatch):
     H = _head_mat_device(g, far_field=True)
     F = factor(H, n, "mixed16", structure=g.factor_segments(), n_positive=n - g.n_vertex_unknowns,
                order=g.factor_order())
-    B = torch.from_numpy(np.random.default_rng(4).standard_normal(n * 48)).cuda()
+    B = torch.from_numpy(np.random.default_rng(4).standard_normal(n * 640)).cuda()
     X = {}
     for mode in ("cache", "none"):
         if mode == "none":
             monkeypatch.setenv("OMH_SOLVE_SCALE_CACHE", "0")
         X[mode] = B.clone()
-        F.solve(X[mode], 48, max_iter=10, tol=1e-12)
-        torch.cuda.synchronize()
+        with Launches() as ran:
+            F.solve(X[mode], 640, max_iter=10, tol=1e-12)
+            torch.cuda.synchronize()
+            split = ran("solve_update_f32s")
+        assert split >= 2 * F.iterations
         monkeypatch.delenv("OMH_SOLVE_SCALE_CACHE", raising=False)
     print("refined with cached scales vs formed each time: max |diff| %.3e after %d passes" % (
         float((X["cache"] - X["none"]).abs().max()), F.iterations), flush=True)

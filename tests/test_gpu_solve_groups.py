@@ -10,6 +10,8 @@ import time
 import numpy as np
 import pytest
 
+from conftest import Launches
+
 pytestmark = pytest.mark.gpu
 
 
@@ -240,10 +242,44 @@ def test_split_products_scale_cache_many_rhs(om, monkeypatch):
         if mode == "none":
             monkeypatch.setenv("OMH_SOLVE_SCALE_CACHE", "0")
         X[mode] = B.clone()
-        F.solve(X[mode], r, max_iter=10, tol=1e-12)
-        torch.cuda.synchronize()
+        with Launches() as ran:
+            F.solve(X[mode], r, max_iter=10, tol=1e-12)
+            torch.cuda.synchronize()
+            split = ran("solve_update_f32s")
+        assert split >= 2 * F.iterations
         monkeypatch.delenv("OMH_SOLVE_SCALE_CACHE", raising=False)
     assert F.iterations >= 2
     assert torch.equal(X["cache"], X["none"])
     res = torch.linalg.norm(B.view(r, n) - X["cache"].view(r, n) @ H.view(n, n)) / torch.linalg.norm(B)
     assert float(res) < 1e-12
+
+
+@pytest.mark.parametrize("order", [False, True])
+@pytest.mark.parametrize("freqs,r", [((9, 8, 6), 37), ((10, 9, 8), 1), ((14, 12, 11), 129), ((9, 9, 9), 200)])
+def test_chunked_residual(om, freqs, r, order):
+    """The FP64 residual of small heads runs in chunks of the inner dimension
+    (uneven segments, odd right-hand sides, a ragged last chunk): the refined
+    solution's own residual, formed by torch, is that of a backward stable
+    FP64 solve."""
+    import torch
+    from openmeeg_amd.api import _head_mat_device, factor
+    from openmeeg_amd import spheres as S
+    meshes = [S.nested_sphere_meshes(f, (R,))[0] for f, R in zip(freqs, (0.87, 0.92, 1.0))]
+    g = om.make_nested_geometry(meshes, (1.0, 0.0125, 1.0))
+    n = g.size
+    H = _head_mat_device(g, far_field=True)
+    F = factor(H, n, "mixed", structure=g.factor_segments(), order=g.factor_order() if order else None)
+    B = torch.from_numpy(np.random.default_rng(n + r).standard_normal((r, n))).cuda()
+    X = B.clone().view(-1)
+    with Launches() as ran:
+        F.solve(X, r, max_iter=20, tol=1e-14)
+        torch.cuda.synchronize()
+        chunks = ran("residual_f64_split")
+    assert chunks > 0 and F.iterations >= 2 and not F.fell_back
+    X, Hm = X.view(r, n), H.view(n, n)
+    res = (X @ Hm - B).norm(dim=1) / (Hm.abs().sum(1).max() * X.norm(dim=1))
+    print("n=%d r=%d: %d chunked products, %d passes, residual %.3e" % (n, r, chunks, F.iterations, float(res.max())),
+          flush=True)
+    # the last correction is below 1e-14 |X|; X and the residual it came from
+    # are rounded in FP64: a few eps |H| |X| a row, sqrt(n) over the rows
+    assert float(res.max()) < 10 * np.sqrt(n) * np.finfo(float).eps
