@@ -122,8 +122,8 @@ __device__ __forceinline__ d3 gauss_point(int order, int i, const d3 P[3]) {
 // atanh and the arc tangent are short polynomials (relative errors 2.7e-17
 // and 3.4e-17); the other waves reduce the atanh's argument first and call
 // atan2 (a lane that satisfies the bounds gets the same bits either way, so
-// that a value does not depend on the lanes beside it).  Roots and reciprocals are the hardware estimates with one cubic
-// Newton step, within about an ulp.
+// that a value does not depend on the lanes beside it).  Roots and reciprocals
+// are the hardware estimates with one cubic Newton step, within about an ulp.
 // ---------------------------------------------------------------------------
 struct AnaTri {            // triangle "analytic side", in registers
     d3 p0, p1, p2, n, e0, e1, e2;

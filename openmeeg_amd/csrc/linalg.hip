@@ -209,8 +209,6 @@ __device__ __forceinline__ int64_t xcd_tile(int64_t b, int64_t per) { return (b 
 __device__ __forceinline__ void map_tile(const TileMap& map, int64_t t, int64_t& tm, int64_t& tn) {
     switch (map.kind) {
         case 1: upper_tile(t, tn, tm); break;   // tn <= tm
-        case 2: tm = map.tm0; tn = t; break;
-        case 3: tn = map.tn0; tm = t; break;
         case 4: lower_band_tile(t, map.ntm, tm, tn); break;
         case 5: full_band_tile(t, map.ntm, map.tn0, tm, tn); break;   // tn0 holds the tile columns
         case 6: {   // lower part of the first tn0 tile columns, row by row
@@ -618,9 +616,10 @@ __global__ void __launch_bounds__(256) k_gemm_grouped(const GemmDesc* __restrict
 // Measured on a 256-block: factor 49 us FP32 and 58 us FP64 (inner panels of
 // 32 columns with LDS products and the trailing part in global memory: 250
 // and 341 us), about 2900 / 3500 cycles a pivot tile and 1000-1500 cycles of
-// barriers and X^T a step; inverse 18 us (45 us FP32, 51 us FP64).  Beside an
-// FP64 update, whose two workgroups a CU leave no room for its registers,
-// the FP64 factor takes 400 us (666 us).
+// barriers and X^T a step; inverse 18 us (45 us FP32, 51 us FP64).  An FP64
+// update's two workgroups a CU leave no room for the FP64 factor's registers:
+// launched beside one it runs when the update drains, so its launch takes as
+// long as the update (up to 13.4 ms at 102408 unknowns).
 // ---------------------------------------------------------------------------
 constexpr int BT = 16;                       // tile of the diagonal block
 constexpr int DF_THREADS = 512;              // factor
@@ -1160,7 +1159,7 @@ __global__ void k_sym_gather(const double* __restrict__ src, int64_t lds, TD* __
 // (rows [dr, dr + h), columns [dc, dc + w) of dst; the diagonal blocks only
 // their lower triangle) is the block of src at rows sr, columns sc: rows are
 // contiguous on both sides, no per-element row map.  Blocks over grid.z,
-// their columns over grid.y (strided), rows over grid.x and the threads.
+// SG_COLS columns each over grid.y, rows over grid.x and the threads.
 constexpr int SG_MAX_BLOCKS = 64;
 // One row and SG_COLS columns of a block a thread, SG_FLY loads in flight (one
 // element a thread and workgroup: 2.9 ms at 17926 unknowns, 38 ms at 102408;
@@ -1191,6 +1190,8 @@ __global__ void __launch_bounds__(256) k_sym_gather_blocks(const double* __restr
     }
 }
 
+// m x n rows: gather dst(i, :) = src(rowmap[i], :), or scatter
+// dst(rowmap[i], :) = src(i, :)
 template <typename TS, typename TD>
 __global__ void k_rows_map(const TS* __restrict__ src, int64_t lds, TD* __restrict__ dst, int64_t ldd, int64_t m,
                            int64_t n, const int32_t* __restrict__ rowmap, int scatter) {
@@ -2305,9 +2306,9 @@ static void launch_tiles(bool ta, bool tb, bool lower, int64_t nblk, TileMap map
 // launch has enough tiles to spread over the XCDs, else the plain order.
 static TileMap l2_map(bool lower, int64_t fm, int64_t fn) {
     const int64_t tiles = lower ? fm * (fm + 1) / 2 : fm * fn;
-    if (tiles < 1024) return lower ? TileMap{1, fm, 0, 0, tiles, 0} : TileMap{0, fm, 0, 0, tiles, 0};
+    if (tiles < 1024) return lower ? TileMap{1, fm, 0, tiles, 0} : TileMap{0, fm, 0, tiles, 0};
     const int64_t per = cdiv(tiles, 8);
-    return lower ? TileMap{4, fm, 0, 0, tiles, per} : TileMap{5, fm, 0, fn, tiles, per};
+    return lower ? TileMap{4, fm, 0, tiles, per} : TileMap{5, fm, fn, tiles, per};
 }
 
 // All tiles of C in one launch.
@@ -2364,7 +2365,7 @@ void build_grouped_gemm(const std::vector<GemmJob>& jobs, bool f32, bool ta, boo
         if (lower && j.m != j.n) throw std::invalid_argument("lower gemm needs a square output");
         const int64_t ntm = cdiv(j.m, TILE), ntn = cdiv(j.n, TILE);
         const bool vec = aligned_bytes(j.A, j.lda, elem) && aligned_bytes(j.B, j.ldb, elem);
-        add(vec ? in : ed, vec ? ti : te, j, TileMap{lower ? 1 : 0, ntm, 0, 0},
+        add(vec ? in : ed, vec ? ti : te, j, TileMap{lower ? 1 : 0, ntm, 0},
             lower ? ntm * (ntm + 1) / 2 : ntm * ntn);
     }
     const int base = (f32 ? 1 : 0) | (ta ? 2 : 0) | (tb ? 4 : 0) | (lower ? 8 : 0) | (wb == 4 ? 16 : 0);
@@ -2552,10 +2553,10 @@ static void splitk_tiles(bool vec, int64_t m, int64_t n, int64_t k, int64_t kc, 
     const dim3 grid((unsigned)(ntm * ntn), nsplit);
     if (vec)
         k_gemm_splitk<T, TA, TB, WB, true><<<grid, 256, 0, st>>>(m, n, k, kc, A, lda, B, ldb, W,
-                                                                 TileMap{0, ntm, 0, 0});
+                                                                 TileMap{0, ntm, 0});
     else
         k_gemm_splitk<T, TA, TB, WB, false><<<grid, 256, 0, st>>>(m, n, k, kc, A, lda, B, ldb, W,
-                                                                  TileMap{0, ntm, 0, 0});
+                                                                  TileMap{0, ntm, 0});
     OMH_LAUNCH_CHECK();
 }
 
@@ -2973,7 +2974,7 @@ static FactorInfo sym_factor_split(float* A, int64_t n, int64_t lda, void* work,
         {
             const int64_t ntm = cdiv(ms, S_TILE), nc = cdiv(w2, S_TILE);
             const int64_t tiles = nc * (nc + 1) / 2 + (ntm - nc) * nc;
-            const TileMap map{6, ntm, 0, nc, tiles, cdiv(tiles, 8)};
+            const TileMap map{6, ntm, nc, tiles, cdiv(tiles, 8)};
             ProfScope ps("factor_strip_f32s", (double)(2 * ms - w2 + 1) * (double)w2 * (double)S_KP, st);
             if (pp)
                 k_syrk_strip<S_KP, true><<<(unsigned)(8 * map.per), 256, 0, st>>>(ms, mp, 0, Ah, Al, Bh, Bl, sc,
@@ -3010,8 +3011,8 @@ static FactorInfo sym_factor_split(float* A, int64_t n, int64_t lda, void* work,
                 if (bf && active_tile_rows(*bf, n, c0, c1, r2, S_TILE, rm, rows)) ntm = rm.c[rm.n];
             }
             const int64_t tiles = ntm * (ntm + 1) / 2;
-            const TileMap map = tiles >= 1024 ? TileMap{4, ntm, 0, 0, tiles, cdiv(tiles, 8)}
-                                              : TileMap{1, ntm, 0, 0, tiles, 0};
+            const TileMap map = tiles >= 1024 ? TileMap{4, ntm, 0, tiles, cdiv(tiles, 8)}
+                                              : TileMap{1, ntm, 0, tiles, 0};
             const unsigned grid = (unsigned)(map.kind == 4 ? 8 * map.per : tiles);
             // 256 x 128 tiles (units of 128 rows, the same remap) while they
             // give at least 4 per CU
@@ -3099,10 +3100,13 @@ FactorInfo sym_factor(T* A, int64_t n, int64_t lda, void* work, hipStream_t st, 
         if (mr > nb2)
             gemm<T>(false, true, false, mr - nb2, nb2, nb, T(-1), X + nb2, ldx, A21, lda, T(1), A22 + nb2, lda, st);
         // factor the next block and form its panel on the side stream (it
-        // touches only the next block's columns, which (b) does not).  Beside
-        // the FP64 update the factor waits for a CU without update workgroups
-        // (0.4 ms instead of 0.06 ms alone), still shorter than the update
-        // while the trailing matrix is large.
+        // touches only the next block's columns, which (b) does not).  The
+        // FP32 block runs beside (b).  The FP64 one waits for a CU without
+        // update workgroups, the first of which (b)'s end leaves, and its
+        // inverse and panel run beside (b)'s edge tiles and after them: at
+        // 102408 unknowns 3.00 s in all, where a block kernel of four waves,
+        // 235 registers and 1.1 ms that ran beside (b) gave 3.04 s, and at
+        // 8136 unknowns 8.1 ms (21.3 ms).
         OMH_HIP(hipEventRecord(la.ready, st));
         OMH_HIP(hipStreamWaitEvent(la.side, la.ready, 0));
         diag_factor<T>(A, lda, e, nb2, Dinv, sgn, info, tiny, la.side);
@@ -4248,9 +4252,9 @@ static SidePool& side_pool() {
 
 // R <- R - H X; with a block structure row segment by row segment, each
 // run of consecutive non-zero column blocks of H in one product.  The row
-// segments write disjoint rows of R and run on up to N_SIDE + 1 streams, so
-// that the last, partly filled round of tiles of one product overlaps the
-// others.
+// segments write disjoint rows of R (their chunks disjoint parts of the
+// scratch) and run on up to N_SIDE + 1 streams, so that the last, partly
+// filled round of tiles of one product overlaps the others.
 // XT (r x n, leading dimension r) = X^T for X n x r (leading dimension ldx):
 // 32 x 32 tiles through LDS, reads and writes along contiguous memory.
 __global__ void __launch_bounds__(256) k_transpose_f64(const double* __restrict__ X, int64_t ldx, int64_t n, int64_t r,
@@ -4276,8 +4280,8 @@ static void residual_update(const double* H, int64_t n, int64_t ldh, const doubl
         return;
     }
     // X^T, so that the segment products are A B^T with contiguous rows of
-    // both operands (the 128 x 128 FP64 tiles); the same sums in the same
-    // order as the products with X
+    // both operands (the 128 x 128 FP64 tiles); whole products sum in the
+    // order of the products with X
     double* XT = (double*)scratch(SCR_RESID_XT, sizeof(double) * (size_t)n * (size_t)r, st);
     k_transpose_f64<<<dim3((unsigned)cdiv(n, 32), (unsigned)cdiv(r, 32)), 256, 0, st>>>(X, ldx, n, r, XT);
     OMH_LAUNCH_CHECK();

@@ -12,12 +12,13 @@ namespace omh {
 constexpr int FACT_NB = 256;   // outer block of the factorisation
 
 // Tile enumeration of a GEMM launch: 0 full grid (ntm row tiles), 1 lower
-// triangle of tiles, 2 one row strip (tile row tm0), 3 one column strip
-// (tile column tn0); 4 and 5: the lower triangle / full grid in an L2-aware
-// order (see map_tile), over a grid of 8 * per workgroups for ntiles tiles.
+// triangle of tiles; 4 and 5: the lower triangle / full grid (tn0 column
+// tiles) in an L2-aware order (see map_tile), over a grid of 8 * per
+// workgroups for ntiles tiles; 6: the lower part of the first tn0 tile
+// columns.
 struct TileMap {
     int kind;
-    int64_t ntm, tm0, tn0;
+    int64_t ntm, tn0;
     int64_t ntiles = 0, per = 0;
 };
 
@@ -83,9 +84,10 @@ struct GemmLaunch {
 };
 
 // Tiles the jobs (all with the same T = float if f32 else double, ta, tb,
-// lower) into descriptors appended to `descs`: an interior launch with
-// unguarded vector loads for the full tiles of aligned products and an edge
-// launch with guarded loads for the rest (the rules of gemm()).
+// lower) into descriptors appended to `descs`: a launch with vector loads
+// for the products with 16-byte aligned operands (clamped loads in their
+// edge tiles) and one with clamped loads for the others (the rules of
+// gemm()).
 void build_grouped_gemm(const std::vector<GemmJob>& jobs, bool f32, bool ta, bool tb, bool lower, int wb,
                         std::vector<GemmDesc>& descs, std::vector<GemmLaunch>& out);
 // Launches l with descriptors at d_descs (device); grid_cap > 0 caps the grid
@@ -140,8 +142,9 @@ void launch_grouped_elem(const ElemDesc* d_descs, int ng, int64_t max_elems, hip
 
 // C = alpha op(A) op(B) + beta C (column-major).  lower: square C, only
 // entries with row >= col are computed (only ta=false, tb=true).
-// prof: optional name under which the interior launch of a lower (SYRK)
-// product is timed (ProfScope name + "_t<tile>").
+// prof: optional name under which a lower (SYRK) product's launch is timed,
+// and of any product the launch over whole 128-wide FP64 tiles (ProfScope
+// name + "_t<tile>").
 template <typename T>
 void gemm(bool ta, bool tb, bool lower, int64_t m, int64_t n, int64_t k, T alpha, const T* A, int64_t lda,
           const T* B, int64_t ldb, T beta, T* C, int64_t ldc, hipStream_t st, const char* prof = nullptr);

@@ -233,7 +233,7 @@ def test_gemm_matches_numpy(om, dtype, ta, tb):
 @pytest.mark.parametrize("ta", [0, 1])
 def test_gemm_large_tile_order(om, dtype, ta):
     """Products with more than 1024 interior tiles run in the XCD-aware,
-    band-swizzled tile order (plus partial edge strips)."""
+    band-swizzled tile order (partial edge tiles in the same launch)."""
     import ctypes as C
     import torch
     from openmeeg_amd import _lib
@@ -342,9 +342,8 @@ def test_fp64_factor_dma_tiles_bitwise(om, monkeypatch):
 
 
 def test_fp64_diag_inverse_narrow_bitwise(om, monkeypatch):
-    """The FP64 diagonal-block inverse on 16-column workgroups (a third of
-    the LDS of the 32-column ones, so that it runs beside the trailing
-    update) sums every entry in the same order: factor and workspace
+    """The FP64 diagonal-block inverse on 16-column workgroups sums every
+    entry in the same order as on 32-column ones: factor and workspace
     (diagonal inverses, signs) bitwise those of the 32-column kernel.  3
     layers of 2562 vertices (n = 17926: a last diagonal block of 6
     columns), with the block structure."""
@@ -642,7 +641,7 @@ def test_split_factor_slice_clock(om, monkeypatch):
 
 def test_split_solve_products(om):
     """The mixed refinement's triangular solves run the products of their
-    full 1024-column groups as split-FP16 MFMA (k_solve_split: the FP32
+    full 1024-column groups as split-FP16 MFMA (k_solve_split_wide: the FP32
     factor over a power-of-two scale per row or column, W's group rows over
     one per column, three FP16 products, FP32 sums).  One solve of the
     refinement (max_iter 1: no correction yet) against the FP32-product solve
