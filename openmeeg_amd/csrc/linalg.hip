@@ -3101,12 +3101,13 @@ FactorInfo sym_factor(T* A, int64_t n, int64_t lda, void* work, hipStream_t st, 
             gemm<T>(false, true, false, mr - nb2, nb2, nb, T(-1), X + nb2, ldx, A21, lda, T(1), A22 + nb2, lda, st);
         // factor the next block and form its panel on the side stream (it
         // touches only the next block's columns, which (b) does not).  The
-        // FP32 block runs beside (b).  The FP64 one waits for a CU without
-        // update workgroups, the first of which (b)'s end leaves, and its
-        // inverse and panel run beside (b)'s edge tiles and after them: at
-        // 102408 unknowns 3.00 s in all, where a block kernel of four waves,
-        // 235 registers and 1.1 ms that ran beside (b) gave 3.04 s, and at
-        // 8136 unknowns 8.1 ms (21.3 ms).
+        // FP32 block runs beside (b): 1.2 ms beside 3.8 ms at 102408
+        // unknowns.  The FP64 one waits for a CU without update workgroups,
+        // the first of which (b)'s end leaves, and its inverse and panel run
+        // beside (b)'s edge tiles and after them: at 102408 unknowns 3.00 s
+        // in all, where a block kernel of four waves, 235 registers and
+        // 1.1 ms that ran beside (b) gave 3.04 s, and at 8136 unknowns
+        // 8.1 ms (21.3 ms).
         OMH_HIP(hipEventRecord(la.ready, st));
         OMH_HIP(hipStreamWaitEvent(la.side, la.ready, 0));
         diag_factor<T>(A, lda, e, nb2, Dinv, sgn, info, tiny, la.side);
